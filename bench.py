@@ -862,7 +862,7 @@ def bench_gemm(ctx, add_flop, timed, g, s, rmap, cta_batch, num_tiles, tpad, T, 
     o1sf = torch.empty((max_tiles * 128, INTER // 32), dtype=torch.uint8, device="cuda")
     o2 = torch.empty((max_tiles * 128, COLS), dtype=torch.bfloat16, device="cuda")
     torch.cuda.synchronize()
-    add_flop("MoE fc1 (MX GEMM + SiTU-GLU + MXFP8)", "kern_k3h_moe_gemm_situ_mx",
+    add_flop("MoE fc1 (MX GEMM + SiTU-GLU + MXFP8)", "kern_k3h_moe_gemm3_situ_mx",
              f"{tpad} rows x {KL} -> 2x{INTER}, E={E}", 2 * tpad * KL * 2 * INTER,
              E * 2 * INTER * (KL // 2 + KL // 32) + tpad * (KL + KL // 32) + tpad * (INTER + INTER // 32),
              timed(lambda: ctx.moe_gemm_mx(ctx.GEMM_SITU_MX, aq, asf, rmap, w13, s13, num_tiles,
@@ -909,7 +909,7 @@ OP_KERNELS = {
     "SiTU landing f32 (n 6144)": ["kern_k3_land_situ"],
     "SiTU landing bf16 (l0, n 33792)": ["kern_k3_situ_bf16"],
     "SiTU landing + latent rms (fused)": ["kern_k3_situ_rms_bf16"],
-    "MoE fc1 (MX GEMM + SiTU-GLU + MXFP8)": ["kern_k3h_moe_gemm_situ_mx"],
+    "MoE fc1 (MX GEMM + SiTU-GLU + MXFP8)": ["kern_k3h_moe_gemm3_situ_mx"],
     "MoE fc2 (MX GEMM, bf16 out)": ["kern_k3h_moe_gemm2_bf16"],
 }
 

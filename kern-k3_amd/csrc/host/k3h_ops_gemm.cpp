@@ -156,6 +156,12 @@ K3H_API int k3h_moe_gemm_mx(k3h_ctx_t ctx, void* stream, int epilogue, const voi
                    epilogue == K3H_GEMM_F32 ? "kern_k3h_moe_gemm2_f32" : "kern_k3h_moe_gemm2_bf16",
                    grid, 1, 1, kBlockWide, stream, args);
   }
+  // fc1 and its f32 tiling: register-weight items where their ring and table fit
+  // (K3B_* of k3_gemm_breg.h: two steps per turn, A scales of K <= 3584; at least four
+  // steps for the loads in flight)
+  if ((epilogue == K3H_GEMM_SITU_MX || epilogue == K3H_GEMM_F32_SITU_TILING) &&
+      K % (2 * kStepK) == 0 && K >= 4 * kStepK && K <= kMaxKNarrow)
+    entry = epilogue == K3H_GEMM_SITU_MX ? "kern_k3h_moe_gemm3_situ_mx" : "kern_k3h_moe_gemm3_acc";
   const uint32_t rows = gemm_grid_rows(max_tiles, N / kTileN);
   if (rows > 65535u) return K3H_EINVAL;
   return k3h_run(ctx, "k3h_moe_gemm", entry, (uint32_t)(N / kTileN), rows, 1, kBlock, stream, args);

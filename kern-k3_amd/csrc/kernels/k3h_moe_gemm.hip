@@ -580,8 +580,8 @@ K3_DEV void k3g_gemm_bf16(K3G_PARAMS, uint16_t* __restrict__ out) {
 // item rather than one per activation (which would cut the unrolled block into
 // a basic block per activation).
 template <int FORM>
-K3_DEV uint32_t k3g_situ_block(const k3_v16f& up, const k3_v16f& gate, float al, float ial,
-                               float be, float ibe, uint8_t* __restrict__ o, int h) {
+K3_DEV uint32_t k3g_situ_codes(const k3_v16f& up, const k3_v16f& gate, float al, float ial,
+                               float be, float ibe, k3_u4& codes) {
   // bf16 activations in q order, as f32; their block amax in f32 (the max of
   // bf16 values is a bf16 value, NaN ignored as in kern_k3_moe_quant)
   float xr[16];
@@ -628,8 +628,16 @@ K3_DEV uint32_t k3g_situ_block(const k3_v16f& up, const k3_v16f& gate, float al,
   uint32_t d0 = c0[0], d1 = c0[1], d2 = c1[0], d3 = c1[1];
   k3g_swap(d0, d2);
   k3g_swap(d1, d3);
-  k3_st16(o + 16 * h, (k3_u4){d0, d2, d1, d3});
+  codes = (k3_u4){d0, d2, d1, d3};
   return (uint32_t)(ex + 127);
+}
+template <int FORM>
+K3_DEV uint32_t k3g_situ_block(const k3_v16f& up, const k3_v16f& gate, float al, float ial,
+                               float be, float ibe, uint8_t* __restrict__ o, int h) {
+  k3_u4 codes;
+  const uint32_t sf = k3g_situ_codes<FORM>(up, gate, al, ial, be, ibe, codes);
+  k3_st16(o + 16 * h, codes);
+  return sf;
 }
 
 template <int KGM>
@@ -720,3 +728,5 @@ K3G_ENTRIES(_w, 224)
 
 #include "k3_gemm_wide.h"
 K3W_ENTRIES
+#include "k3_gemm_breg.h"
+K3B_ENTRIES

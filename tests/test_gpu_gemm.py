@@ -289,3 +289,43 @@ def test_wide_items_match_4wave(ctx, K):
             same = torch.equal(got.view(torch.uint8), fc1t.view(torch.uint8))
             print(f"  kern_k3h_moe_gemm_situ_acc: identical = {same}", flush=True)
             assert same
+
+
+@pytest.mark.parametrize("K", [512, 768, 3584])
+def test_repeated_rows_match_gathered(ctx, K):
+    """Tiles padded by repeating a row index (the fc1 kernel computes one or two m tiles
+    and repeats the last row's results) against the same rows gathered beforehand
+    (a_rows = None, every row computed), bit for bit: distinct rows on both sides of each
+    m tile's edge, a repeat of a live row's index, and index -1 (row 0)."""
+    E, inter = 3, 256
+    N = 2 * inter
+    _case(f"repeated rows E={E} inter={inter} K={K}")
+    g, q, sf, w, wsf = _inputs(7900 + K, 300, E, N, K, wsf_range=(121, 126))
+    lives = [1, 2, 30, 31, 32, 33, 62, 63, 64, 65, 96, 127, 128]
+    rows = np.zeros((len(lives) + 2, 128), np.int32)
+    for i, n in enumerate(lives):
+        rows[i, :n] = 1 + g.permutation(299)[:n]
+    rows[-2] = -1
+    rows[-1, :40], rows[-1, 40:] = 1 + np.arange(40), 7
+    cta = g.integers(0, E, len(rows)).astype(np.int32)
+    nt = len(rows)
+    src = np.maximum(rows, 0).reshape(-1)
+    wt, st = _tiled(ctx, w, wsf, E, N, K, 1)
+    alpha, beta = to_dev(np.full(E, 4.0, np.float32)), to_dev(np.full(E, 25.0, np.float32))
+    dnt, dcta = to_dev(np.array([nt], np.int32)), to_dev(cta)
+    got = []
+    for a, asf, idx in ((q, sf, to_dev(rows.reshape(-1))), (q[src], sf[src], None)):
+        acc = torch.full((nt * 128, N), float("nan"), device="cuda")
+        # scale bytes 2-byte aligned in one case, 4-byte aligned in the other
+        osf = torch.full((nt * 128 * (inter // 32) + 2,), 0x5a, dtype=torch.uint8, device="cuda")
+        osf = osf[2:] if idx is None else osf[:-2]
+        oq = torch.full((nt * 128, inter), 0x5a, dtype=torch.uint8, device="cuda")
+        da, dasf = to_dev(a), to_dev(asf)
+        ctx.moe_gemm_mx(ctx.GEMM_F32_SITU_TILING, da, dasf, idx, wt, st, dnt, dcta, nt, E, N, K, acc)
+        ctx.moe_gemm_mx(ctx.GEMM_SITU_MX, da, dasf, idx, wt, st, dnt, dcta, nt, E, N, K, oq, osf,
+                        alpha, beta)
+        torch.cuda.synchronize()
+        got.append((from_dev(acc).view(np.uint32), from_dev(oq), from_dev(osf)))
+    for name, x, y in zip(("accumulators", "codes", "scales"), *got):
+        bad = (x.reshape(nt, -1) != y.reshape(nt, -1)).any(1)
+        assert not bad.any(), f"{name}: tiles {np.flatnonzero(bad)} differ"
