@@ -203,7 +203,9 @@ K3H_API int k3h_moe_quant(k3h_ctx_t ctx, void* stream, const void* x, void* q, v
  * k3_quant_fp8_pair_v2.cu:42,63; manifest op quant_fp8_tensor, json:407194):
  * partials[nb] f32 (scratch owned by the caller), scale_out[1] f32, y u8 [n].
  * Both launches grid (nb), block 256; the manifest uses nb = 2048.  v2 != 0
- * selects the _v2 module.  The amax and apply steps are also exported alone. */
+ * selects the _v2 module.  The amax and apply steps are also exported alone.  At
+ * nb = 2048 and n >= 24 << 20 the v2 call runs k3h_quant_fp8_mark and
+ * k3h_quant_fp8_once (256 workgroups, one per CU) instead, with the same outputs. */
 K3H_API int k3h_quant_fp8_amax(k3h_ctx_t ctx, void* stream, int v2, const void* x, int n,
                                float* partials, int nb);
 K3H_API int k3h_quant_fp8_apply(k3h_ctx_t ctx, void* stream, int v2, const void* x, void* y,

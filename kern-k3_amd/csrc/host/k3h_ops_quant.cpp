@@ -4,6 +4,13 @@
 
 namespace {
 const char* quant_key(int v2) { return v2 ? "k3_quant_fp8_pair_v2" : "k3_quant_fp8_pair"; }
+// k3h_quant_fp8_once (one launch that keeps most of x on the chip between the passes): one
+// workgroup per CU, the manifest's nb only.
+constexpr int kOnceNb = 2048, kOnceGrid = 256, kOnceBlock = 1024;
+// below, its fixed cost exceeds the second read of x (20.9 -> 18.4 us at n = 25 M, 15.2 ->
+// 16.7 us at 18 M)
+constexpr int kOnceMinN = 24 << 20;
+constexpr int kOnceSpinTicks = 20000;  // 200 us of the 100 MHz clock
 bool quant_args_ok(const void* x, int n, const void* partials, int nb) {
   return n >= 0 && nb >= 1 && nb <= 65535 && k3h_okp(x, 16) && k3h_okp(partials, 4);
 }
@@ -32,6 +39,24 @@ K3H_API int k3h_quant_fp8_apply(k3h_ctx_t ctx, void* stream, int v2, const void*
 
 K3H_API int k3h_quant_fp8_tensor(k3h_ctx_t ctx, void* stream, int v2, const void* x, void* y,
                                  float* scale_out, float* partials, int n, int nb) {
+  if (!ctx || !quant_args_ok(x, n, partials, nb) || !k3h_okp(y, 8) ||
+      (scale_out && !k3h_aligned(scale_out, 4)))
+    return K3H_EINVAL;
+  if (v2 && nb == kOnceNb && n >= kOnceMinN) {
+    int hold = 0;
+    const int rc = k3h_ctx_resident(ctx, quant_key(1), "k3h_quant_fp8_once", kOnceBlock, &hold);
+    if (rc != K3H_OK) return rc;
+    if (hold >= kOnceGrid) {  // the whole grid at once, as the wait for the partials assumes
+      K3hArgs m;
+      m.ptr(partials);
+      const int r = k3h_run(ctx, quant_key(1), "k3h_quant_fp8_mark", kOnceNb / kOnceBlock, 1, 1,
+                            kOnceBlock, stream, m);
+      if (r != K3H_OK) return r;
+      K3hArgs a;
+      a.ptr(x).ptr(y).i32(n).ptr(partials).ptr(scale_out).i32(kOnceSpinTicks);
+      return k3h_run(ctx, quant_key(1), "k3h_quant_fp8_once", kOnceGrid, 1, 1, kOnceBlock, stream, a);
+    }
+  }
   const int r = k3h_quant_fp8_amax(ctx, stream, v2, x, n, partials, nb);
   if (r != K3H_OK) return r;
   return k3h_quant_fp8_apply(ctx, stream, v2, x, y, n, partials, nb, scale_out);

@@ -137,3 +137,257 @@ extern "C" __global__ void __launch_bounds__(QT) K3_APPLY_NAME(
     y[e] = (uint8_t)(k3_pack_e4m3x2(k3_bf(x[e]) * inv, 0.0f) & 0xffu);
   }
 }
+
+#ifdef K3_QUANT_V2
+// One pass over HBM for large tensors: k3h_quant_fp8_mark, then k3h_quant_fp8_once, with
+// the outputs of the pair at nb = 2048 bit for bit (partials included).  The pair reads
+// x twice, and although the second pass comes from the MALL it costs as much as the
+// first.  Here one persistent launch (256 workgroups of 1024 threads, one per CU) keeps
+// the last 24 of a thread's vectors on the chip (15 in registers, 9 in LDS: 98 MB of
+// x in all), meets at the partials, and quantises what it holds; only the vectors before
+// those are read again, from the MALL.  Quarter s of workgroup g plays the pair's blocks
+// 8 g + s and 8 g + 4 + s, so a thread's m-th vector is vector
+// (8 g + 4 (m & 1) + s + 2048 (m >> 1)) * 256 + t and the chip sweeps x front to back.
+// Measured over three rotating sets: n = 117 M 87.2 -> 74.8 us, 59 M 44.9 -> 33.7, 29 M
+// 23.9 -> 19.5, 25 M 20.9 -> 18.4, 18 M 15.2 -> 16.7 (mark, dispatch and the meeting cost
+// about 13 us): the host takes it for n >= 24 << 20.  At 117 M a workgroup spends 36 us
+// reading (6.5 TB/s), 4 us meeting and 20 us on the second pass.
+// Requires n >= 8.
+#define QO_NB 2048
+#define QO_REG 15           // vectors a thread keeps in registers
+#define QO_LDS 9            // and in LDS
+#define QO_HELD (QO_REG + QO_LDS)
+#define QO_UNSET 0xffffffffu  // a partial is a non-negative bf16 pattern << 16
+
+extern "C" __global__ void __launch_bounds__(1024) k3h_quant_fp8_mark(uint32_t* __restrict__ partials) {
+  partials[blockIdx.x * 1024 + threadIdx.x] = QO_UNSET;
+}
+
+K3_DEV uint32_t k3_qo_max(uint32_t m, k3_u4 v) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t a = v[j] & 0x7fff7fffu;
+    const uint32_t lo = a & 0xffffu, hi = a >> 16;
+    m = m > lo ? m : lo;
+    m = m > hi ? m : hi;
+  }
+  return m;
+}
+K3_DEV k3_u2 k3_qo_codes(k3_u4 v, float inv) {
+  k3_u2 o;
+  o[0] = k3_pack_e4m3x4(k3_bf_lo(v[0]) * inv, k3_bf_hi(v[0]) * inv, k3_bf_lo(v[1]) * inv,
+                        k3_bf_hi(v[1]) * inv);
+  o[1] = k3_pack_e4m3x4(k3_bf_lo(v[2]) * inv, k3_bf_hi(v[2]) * inv, k3_bf_lo(v[3]) * inv,
+                        k3_bf_hi(v[3]) * inv);
+  return o;
+}
+K3_DEV uint32_t k3_qo_wave_max(uint32_t m) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint32_t p = (uint32_t)__shfl_xor((int)m, o, 64);
+    m = m > p ? m : p;
+  }
+  return m;
+}
+
+extern "C" __global__ void __launch_bounds__(1024) k3h_quant_fp8_once(
+    const uint16_t* __restrict__ x, uint8_t* __restrict__ y, int n, uint32_t* __restrict__ partials,
+    float* __restrict__ scale_out, int spin_ticks) {
+  __shared__ k3_u4 held[QO_LDS][1024];
+  __shared__ uint32_t red[2][16];
+  const int tid = threadIdx.x, t = tid & 255, s = tid >> 8, wave = tid >> 6;
+  const int b0 = 8 * (int)blockIdx.x + s;
+  const long long nv = n >> 3;
+  const k3_u4 zero = {0, 0, 0, 0};
+  // slot m's vector of this thread (n < 2^31, so an index fits 32 bits); slots past
+  // the end read the last vector and count as zero
+  const uint32_t last = (uint32_t)nv - 1;
+  auto vec = [&](int m) -> uint32_t {
+    return (8u * blockIdx.x + 4u * (uint32_t)(m & 1) + (uint32_t)QO_NB * (uint32_t)(m >> 1)) * 256u +
+           (uint32_t)tid;
+  };
+  auto at = [&](uint32_t i) { return (const k3_u4*)((const uint8_t*)x + 16u * (size_t)i); };
+  auto hold = [&](int m) {
+    const uint32_t i = vec(m);
+    return __builtin_nontemporal_load(at(i < last ? i : last));
+  };
+  auto live = [&](int m, k3_u4 v) { return vec(m) <= last ? v : zero; };
+  auto put = [&](uint32_t i, k3_u4 v, float inv) { k3_st8_nt(y + 8u * (size_t)i, k3_qo_codes(v, inv)); };
+  const int steps = (int)((nv + (long long)QO_NB * 256 - 1) / ((long long)QO_NB * 256));
+  const int M = 2 * steps;                             // vector slots (the last two may be past the end)
+  const int S = M > QO_HELD ? M - QO_HELD : 0;         // the first S are read again
+  uint32_t mx0 = 0, mx1 = 0;
+  // S is even (M and QO_HELD are)
+  // the slots read again (cacheable, so that they stay in the MALL), four by four with
+  // the next four in flight; slots past S repeat the last pair
+  auto again = [&](int m) { return vec(m < S ? m : S - 2 + (m & 1)); };
+  k3_u4 v[2][4];
+  if (S > 0) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[0][k] = *at(again(k));
+    for (int m = 0; m < S; m += 8) {
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[1 - half][k] = *at(again(m + 4 * half + 4 + k));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < 4; k += 2) {
+          mx0 = k3_qo_max(mx0, v[half][k]);
+          mx1 = k3_qo_max(mx1, v[half][k + 1]);
+        }
+      }
+    }
+  }
+  {
+    k3_u4 l[QO_LDS];
+#pragma unroll
+    for (int k = 0; k < QO_LDS; ++k) {
+      l[k] = hold(S + k);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < QO_LDS; ++k) {
+      l[k] = live(S + k, l[k]);
+      if (k & 1) mx1 = k3_qo_max(mx1, l[k]);
+      else mx0 = k3_qo_max(mx0, l[k]);
+      held[k][tid] = l[k];
+    }
+  }
+  k3_u4 r[QO_REG];
+#pragma unroll
+  for (int k = 0; k < QO_REG; ++k) {
+    r[k] = hold(S + QO_LDS + k);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int k = 0; k < QO_REG; ++k) {
+    r[k] = live(S + QO_LDS + k, r[k]);
+    if ((QO_LDS + k) & 1) mx1 = k3_qo_max(mx1, r[k]);
+    else mx0 = k3_qo_max(mx0, r[k]);
+  }
+  if (b0 == 0 && t < (n & 7)) {  // the n % 8 tail belongs to block 0
+    const uint32_t a = x[nv * 8 + t] & 0x7fffu;
+    mx0 = mx0 > a ? mx0 : a;
+  }
+  mx0 = k3_qo_wave_max(mx0);
+  mx1 = k3_qo_wave_max(mx1);
+  if ((tid & 63) == 0) {
+    red[0][wave] = mx0;
+    red[1][wave] = mx1;
+  }
+  __syncthreads();
+  if (tid < 8) {
+    const uint32_t* q = &red[tid >> 2][4 * (tid & 3)];
+    uint32_t b = q[0];
+#pragma unroll
+    for (int k = 1; k < 4; ++k) b = b > q[k] ? b : q[k];
+    __hip_atomic_store(partials + 8 * blockIdx.x + tid, b << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  // the first slots read again are requested before the wait
+  if (S > 0) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[0][k] = __builtin_nontemporal_load(at(again(k)));
+  }
+  // every block's partial: poll until it is set, for spin_ticks (10 ns each) at most
+  uint32_t p0, p1;
+  {
+    const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
+    for (;;) {
+      p0 = __hip_atomic_load(partials + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      p1 = __hip_atomic_load(partials + 1024 + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (__ballot(p0 == QO_UNSET || p1 == QO_UNSET) == 0) break;
+      if ((uint64_t)__builtin_amdgcn_s_memrealtime() - t0 >= (uint64_t)spin_ticks) break;
+      __builtin_amdgcn_s_sleep(1);
+    }
+  }
+  // the max over the partials that are not NaN patterns (those compare as bits in
+  // `partials`, and the scale ignores them)
+  auto fold = [&](float f, uint32_t p) { return p == QO_UNSET ? f : __builtin_fmaxf(f, __uint_as_float(p)); };
+  float amax = fold(fold(0.0f, p0), p1);
+  __shared__ float fred[16];
+  __shared__ int missing[16];
+  {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) amax = __builtin_fmaxf(amax, __shfl_xor(amax, o, 64));
+    const bool miss = __ballot(p0 == QO_UNSET || p1 == QO_UNSET) != 0;
+    if ((tid & 63) == 0) {
+      fred[wave] = amax;
+      missing[wave] = miss;
+    }
+  }
+  __syncthreads();
+  bool any = false;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    amax = __builtin_fmaxf(amax, fred[k]);
+    any |= missing[k] != 0;
+  }
+  if (any) {
+    // A workgroup that is not resident yet cannot have set its partials (the device is
+    // shared): the waiting ones take the missing blocks' maxima themselves, each starting
+    // at another block and storing what it finds for the others, so no workgroup ever
+    // depends on another one running.
+    for (int c = 0; c < QO_NB; ++c) {
+      const int b = (c + 8 * (int)blockIdx.x) & (QO_NB - 1);
+      __syncthreads();
+      if (tid == 0)
+        red[1][0] = __hip_atomic_load(partials + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __syncthreads();
+      uint32_t p = red[1][0];  // the same for the whole workgroup
+      if (p == QO_UNSET) {
+        uint32_t bm = 0;
+        for (long long i = (b + (long long)QO_NB * s) * 256 + t; i < nv; i += 4LL * QO_NB * 256)
+          bm = k3_qo_max(bm, k3_ld16(x + i * 8));
+        if (b == 0 && tid < (n & 7)) {
+          const uint32_t a = x[nv * 8 + tid] & 0x7fffu;
+          bm = bm > a ? bm : a;
+        }
+        bm = k3_qo_wave_max(bm);
+        if ((tid & 63) == 0) red[0][wave] = bm;
+        __syncthreads();
+#pragma unroll
+        for (int v = 0; v < 16; ++v) bm = bm > red[0][v] ? bm : red[0][v];
+        p = bm << 16;
+        if (tid == 0)
+          __hip_atomic_store(partials + b, p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      }
+      amax = __builtin_fmaxf(amax, __uint_as_float(p));
+    }
+  }
+  const float scale = amax > 0.0f ? amax / 448.0f : 1.0f;
+  if (blockIdx.x == 0 && tid == 0 && scale_out) *scale_out = scale;
+  const float inv = 1.0f / scale;
+  uint32_t tid2 = (uint32_t)tid;
+  asm volatile("" : "+v"(tid2));  // no address is kept across the wait
+  auto vec2 = [&](int m) { return vec(m) - (uint32_t)tid + tid2; };
+
+  // the held vectors, then the ones read again
+#pragma unroll
+  for (int k = 0; k < QO_REG; ++k) {
+    const uint32_t i = vec2(S + QO_LDS + k);
+    if (i <= last) put(i, r[k], inv);
+  }
+#pragma unroll
+  for (int k = 0; k < QO_LDS; ++k) {
+    const uint32_t i = vec2(S + k);
+    if (i <= last) put(i, held[k][tid], inv);
+  }
+  for (int m = 0; m < S; m += 8) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        v[1 - half][k] = __builtin_nontemporal_load(at(again(m + 4 * half + 4 + k)));
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (m + 4 * half + k < S) put(vec(m + 4 * half + k), v[half][k], inv);
+    }
+  }
+  if (b0 == 0 && t < (n & 7)) {
+    const long long e = nv * 8 + t;
+    y[e] = (uint8_t)(k3_pack_e4m3x2(k3_bf(x[e]) * inv, 0.0f) & 0xffu);
+  }
+}
+#endif  // K3_QUANT_V2

@@ -1,5 +1,6 @@
 """GPU parity: per-tensor fp8 pair (v1 and v2 modules) against the C oracle,
 bit-exact for the partials, the scale and every e4m3 byte."""
+import ctypes
 import json
 import os
 
@@ -86,3 +87,64 @@ def test_quant_fp8_manifest_op(ctx):
     assert np.array_equal(from_dev(p), want_p)
     assert from_dev(s)[0] == want_s[0]
     assert np.array_equal(from_dev(y), want_y)
+
+
+def _once(ctx, x, n, spin_ticks):
+    """k3h_quant_fp8_mark + k3h_quant_fp8_once launched directly: (y, scale, partials)."""
+    y = torch.full((n + 8,), 0x5a, dtype=torch.uint8, device="cuda")
+    s = torch.zeros(1, dtype=torch.float32, device="cuda")
+    p = torch.zeros(2048, dtype=torch.float32, device="cuda")
+    key, stream = "k3_quant_fp8_pair_v2", torch.cuda.current_stream().cuda_stream
+    for entry, grid, kinds, vals in (
+            ("k3h_quant_fp8_mark", 2, ["buffer"], [p]),
+            ("k3h_quant_fp8_once", 256, ["buffer", "buffer", "i32", "buffer", "buffer", "i32"],
+             [x, y, n, p, s, spin_ticks])):
+        buf = k3h.pack_args(kinds, vals)
+        cbuf = ctypes.create_string_buffer(buf, len(buf))
+        k3h._check(ctx.L.k3h_launch(ctx.function(key, entry), (ctypes.c_uint32 * 3)(grid, 1, 1),
+                                    (ctypes.c_uint32 * 3)(1024, 1, 1), 0, stream,
+                                    ctypes.cast(cbuf, ctypes.c_void_p), len(buf)), entry)
+    torch.cuda.synchronize()
+    return y, s, p
+
+
+@pytest.mark.parametrize("n,spin", [(4096, 20000), (24 << 20, 20000), (12 << 22, 20000),
+                                    ((12 << 22) + 7, 20000), ((12 << 22) + 8, 20000),
+                                    ((15 << 22) + 4099, 20000), ((30 << 20) + 13, 0)])
+def test_quant_fp8_one_launch(ctx, n, spin):
+    """The one-launch form against the amax / apply entries, bit for bit: tensors that fit
+    the chip, that fill it exactly (24 vectors per thread) and that are partly read again;
+    NaN and -inf among the inputs; with no wait at all (spin 0) every workgroup takes the
+    maxima it misses itself."""
+    print(f"[case] quant_fp8 one launch n={n} spin={spin}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(1300 + n % 97)
+    x = torch.empty(n, device="cuda").normal_(0, 2, generator=g).to(torch.bfloat16)
+    x[n // 3], x[n - 1], x[n // 2] = float("nan"), -300.0, -0.0
+    nb = 2048
+    want_y = torch.full((n + 8,), 0x5a, dtype=torch.uint8, device="cuda")
+    want_s = torch.zeros(1, dtype=torch.float32, device="cuda")
+    want_p = torch.empty(nb, dtype=torch.float32, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    assert ctx.L.k3h_quant_fp8_amax(ctx.h, stream, 1, x.data_ptr(), n, want_p.data_ptr(), nb) == 0
+    assert ctx.L.k3h_quant_fp8_apply(ctx.h, stream, 1, x.data_ptr(), want_y.data_ptr(), n,
+                                     want_p.data_ptr(), nb, want_s.data_ptr()) == 0
+    y, s, p = _once(ctx, x, n, spin)
+    assert torch.equal(p.view(torch.int32), want_p.view(torch.int32))
+    assert s.view(torch.int32).item() == want_s.view(torch.int32).item()
+    assert torch.equal(y, want_y)
+
+
+@pytest.mark.parametrize("n", [(24 << 20) - 1, 24 << 20, (24 << 20) + 5])
+def test_quant_fp8_tensor_route(ctx, n):
+    """The typed call on both sides of the size where it changes to the one-launch form."""
+    print(f"[case] quant_fp8_tensor route n={n}", flush=True)
+    x = normal_bf16(rng(1400), (n,), outlier_p=0.001)
+    want_p = O.quant_fp8_amax(x, n, 2048, v2=True)
+    want_y, want_s = O.quant_fp8_apply(x, n, want_p, 2048)
+    y = torch.empty(n + 8, dtype=torch.uint8, device="cuda")
+    s = torch.empty(1, dtype=torch.float32, device="cuda")
+    p = torch.empty(2048, dtype=torch.float32, device="cuda")
+    ctx.quant_fp8_tensor(to_dev(x), y, s, p, n)
+    torch.cuda.synchronize()
+    assert np.array_equal(from_dev(p), want_p) and from_dev(s)[0] == want_s[0]
+    assert np.array_equal(from_dev(y)[:n], want_y)
