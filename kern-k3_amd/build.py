@@ -171,6 +171,26 @@ def build_host() -> str:
     return dst
 
 
+def build_py() -> str:
+    """The Python extension of k3h.py's tensor checks (host code, torch's C++ headers)."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    dst = os.path.join(OUT, "_k3h_py.so")
+    tmp = dst + ".tmp"
+    tlib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(x for p in (sysconfig.get_paths()["include"], *cpp_extension.include_paths())
+             for x in ("-isystem", p)),
+           "-o", tmp, os.path.join(CSRC, "host", "k3h_py.cpp"),
+           "-L", tlib, "-ltorch_python", "-ltorch_cpu", "-lc10", f"-Wl,-rpath,{tlib}"]
+    _run(cmd, "_k3h_py.so")
+    os.replace(tmp, dst)
+    return dst
+
+
 def build_oracle() -> str | None:
     odir = os.path.join(REPO, "oracle")
     if not os.path.exists(os.path.join(odir, "Makefile")):
@@ -198,6 +218,7 @@ def build(jobs: int | None = None, only: list[str] | None = None, oracle: bool =
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
         futs = [ex.submit(build_module, k) for k in keys]
         futs.append(ex.submit(build_host))
+        futs.append(ex.submit(build_py))
         if oracle:
             futs.append(ex.submit(build_oracle))
         for f in futs:

@@ -9,6 +9,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <string_view>
 #include <tuple>
 #include <utility>
 
@@ -103,11 +104,22 @@ K3H_API int k3h_runtime_version(int* version) {
 }  // extern "C"
 
 // ---------------------------------------------------------------- context
+// (module key, entry) order over strings and views alike, so that a lookup builds no
+// string (every launch makes one).
+struct K3hEntryLess {
+  using is_transparent = void;
+  template <class A, class B>
+  bool operator()(const A& a, const B& b) const {
+    const int c = std::string_view(a.second).compare(b.second);
+    return c != 0 ? c < 0 : std::string_view(a.first) < std::string_view(b.first);
+  }
+};
+
 struct k3h_ctx_s {
   std::string dir;
   std::mutex mu;
   std::map<std::string, k3h_module_t> mods;
-  std::map<std::pair<std::string, std::string>, k3h_fn_t> fns;
+  std::map<std::pair<std::string, std::string>, k3h_fn_t, K3hEntryLess> fns;
   // (function, block size, device) -> workgroups the device holds at once
   std::map<std::tuple<k3h_fn_t, uint32_t, int>, int> resident;
 };
@@ -162,9 +174,10 @@ K3H_API int k3h_ctx_function(k3h_ctx_t ctx, const char* module_key, const char* 
                              k3h_fn_t* out) {
   if (!ctx || !module_key || !entry || !out) return K3H_EINVAL;
   std::lock_guard<std::mutex> lock(ctx->mu);
-  const auto key = std::make_pair(std::string(module_key), std::string(entry));
-  auto it = ctx->fns.find(key);
+  const auto it = ctx->fns.find(
+      std::pair<std::string_view, std::string_view>(module_key, entry));
   if (it != ctx->fns.end()) { *out = it->second; return K3H_OK; }
+  const auto key = std::make_pair(std::string(module_key), std::string(entry));
   k3h_module_t m = nullptr;
   auto mi = ctx->mods.find(key.first);
   if (mi == ctx->mods.end()) {

@@ -17,6 +17,7 @@ gfx950 code object.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import struct
 from typing import Any, Sequence
@@ -159,36 +160,31 @@ def _check(rc: int, what: str) -> None:
 
 
 # ---------------------------------------------------------------- tensor checks
-def _ptr(t: torch.Tensor | None) -> int | None:
-    return None if t is None else t.data_ptr()
+def _load_checks():
+    """The extension built beside the library (csrc/host/k3h_py.cpp)."""
+    path = os.path.join(BUILD, "_k3h_py.so")
+    if not os.path.exists(path):
+        raise FileNotFoundError(f"{path} is missing: build it with `python kern-k3_amd/build.py`")
+    spec = importlib.util.spec_from_file_location("_k3h_py", path)
+    m = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(m)
+    return m
 
 
-def _dev(t: torch.Tensor, name: str, dtypes: Sequence[torch.dtype], numel: int | None = None,
-         align: int = 16) -> None:
-    if not isinstance(t, torch.Tensor):
-        raise ValueError(f"{name}: expected a torch tensor")
-    if t.device.type != "cuda":
-        raise ValueError(f"{name}: must be a GPU tensor (got {t.device})")
-    if t.dtype not in dtypes:
-        raise ValueError(f"{name}: dtype {t.dtype} not in {list(dtypes)}")
-    if not t.is_contiguous():
-        raise ValueError(f"{name}: must be contiguous")
-    if numel is not None and t.numel() < numel:
-        raise ValueError(f"{name}: needs at least {numel} elements, has {t.numel()}")
-    if t.data_ptr() % align:
-        raise ValueError(f"{name}: must be {align}-byte aligned")
-
-
-BF16 = (torch.bfloat16,)
-U8 = (torch.uint8, torch.float8_e4m3fn)
-F32 = (torch.float32,)
-I32 = (torch.int32,)
-I64 = (torch.int64,)
+_py = _load_checks()
+# _dev(t, name, dtypes, numel=None, align=16) raises ValueError for anything but a
+# contiguous GPU tensor of one of dtypes (a sum of the masks below), at least numel
+# elements and align-byte aligned; _ptr(t) is its address (None for None)
+_dev, _ptr = _py.dev, _py.ptr
+BF16, F32, U8, I32, I64, ANY = _py.BF16, _py.F32, _py.U8, _py.I32, _py.I64, _py.ANY
 
 
 def _stream(stream: Any) -> int | None:
     if stream is None:
-        return torch.cuda.current_stream().cuda_stream
+        if not torch.cuda.is_initialized():
+            return torch.cuda.current_stream().cuda_stream
+        # the current stream's handle without a Stream object
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
     if isinstance(stream, int):
         return stream
     return stream.cuda_stream
@@ -625,7 +621,7 @@ class Ctx:
         inner = 3072
         _dev(partial, "partial", BF16, 4 * inner)
         _dev(cw, "cw", F32, 12 * inner)
-        _dev(kda_base, "kda_base", (kda_base.dtype,))
+        _dev(kda_base, "kda_base", ANY)
         _dev(line_index, "line_index", I32, 1, align=4)
         _dev(wsm_partial, "wsm_partial", F32, 256)
         for nm, t in (("span_q", span_q), ("span_k", span_k), ("span_v", span_v)):
@@ -742,8 +738,8 @@ class Ctx:
         nbytes = src.numel() * src.element_size()
         if nbytes % 16 or dst.numel() * dst.element_size() < nbytes:
             raise ValueError("stream_copy: size must be a multiple of 16 bytes and fit dst")
-        _dev(src, "src", (src.dtype,))
-        _dev(dst, "dst", (dst.dtype,))
+        _dev(src, "src", ANY)
+        _dev(dst, "dst", ANY)
         _check(self.L.k3h_stream_copy(self.h, _stream(stream), _ptr(src), _ptr(dst), nbytes // 16),
                "stream_copy")
 
