@@ -143,6 +143,17 @@ K3H_API int k3h_moe_gemm_mx(k3h_ctx_t ctx, void* stream, int epilogue, const voi
       return K3H_EINVAL;
   }
   if (max_tiles == 0) return K3H_OK;
+  // register-weight items (k3_gemm_breg.h) where their A ring and scale table fit: two steps
+  // per turn, at least four steps for the loads in flight, A scales of K <= 3584
+  const bool breg = K % (2 * kStepK) == 0 && K >= 4 * kStepK && K <= kMaxKNarrow;
+  const uint32_t rows = gemm_grid_rows(max_tiles, N / kTileN);
+  // bf16 with hardly a row per expert (max_tiles counts a partial tile for each): the
+  // weights' stream bounds it, and 256-column items on two workgroups per CU stream them
+  // faster as long as they fit about one round (1 tile 29 -> 22 us, 39 tiles 86 -> 71, but 56
+  // tiles 93 -> 98)
+  if (epilogue == K3H_GEMM_BF16 && breg && max_tiles <= E + E / 16 && rows <= 65535u)
+    return k3h_run(ctx, "k3h_moe_gemm", "kern_k3h_moe_gemm3_bf16", (uint32_t)(N / kTileN), rows, 1,
+                   kBlock, stream, args);
   // f32 / bf16 epilogues on 512-column items: persistent 8-wave workgroups
   // (kern_k3h_moe_gemm2_*, one per CU, grid a multiple of the 8 XCDs) where the
   // shape allows them; else, and for the SiTU-GLU + MXFP8 epilogue and its f32 tiling, 256-column
@@ -156,14 +167,9 @@ K3H_API int k3h_moe_gemm_mx(k3h_ctx_t ctx, void* stream, int epilogue, const voi
                    epilogue == K3H_GEMM_F32 ? "kern_k3h_moe_gemm2_f32" : "kern_k3h_moe_gemm2_bf16",
                    grid, 1, 1, kBlockWide, stream, args);
   }
-  // fc1 and its f32 tiling: register-weight items where their ring and table fit
-  // (K3B_* of k3_gemm_breg.h: two steps per turn, A scales of K <= 3584; at least four
-  // steps for the loads in flight)
-  if ((epilogue == K3H_GEMM_SITU_MX || epilogue == K3H_GEMM_F32_SITU_TILING) &&
-      K % (2 * kStepK) == 0 && K >= 4 * kStepK && K <= kMaxKNarrow)
-    entry = epilogue == K3H_GEMM_SITU_MX ? "kern_k3h_moe_gemm3_situ_mx" : "kern_k3h_moe_gemm3_acc";
-  const uint32_t rows = gemm_grid_rows(max_tiles, N / kTileN);
   if (rows > 65535u) return K3H_EINVAL;
+  if (breg && epilogue == K3H_GEMM_SITU_MX) entry = "kern_k3h_moe_gemm3_situ_mx";
+  if (breg && epilogue == K3H_GEMM_F32_SITU_TILING) entry = "kern_k3h_moe_gemm3_acc";
   return k3h_run(ctx, "k3h_moe_gemm", entry, (uint32_t)(N / kTileN), rows, 1, kBlock, stream, args);
 }
 

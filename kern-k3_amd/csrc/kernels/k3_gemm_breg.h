@@ -1,9 +1,9 @@
 // Register-weight items for the MoE expert GEMMs (module k3h_moe_gemm, included by
 // k3h_moe_gemm.hip after the 256-column kernels and k3_gemm_wide.h, whose layouts,
-// item split and helpers it shares).  Entries kern_k3h_moe_gemm3_situ_mx (fc1) and
-// kern_k3h_moe_gemm3_acc (its tiling with f32 output): the same products as the
-// 256-column kernels bit for bit (the same MFMA sequence per output element), for
-// 512 <= K <= 3584, K % 256 == 0.
+// item split and helpers it shares).  Entries kern_k3h_moe_gemm3_situ_mx (fc1),
+// kern_k3h_moe_gemm3_acc (its tiling with f32 output) and kern_k3h_moe_gemm3_bf16 (fc2 over
+// few tiles): the same products as the 256-column kernels bit for bit (the same MFMA
+// sequence per output element), for 512 <= K <= 3584, K % 256 == 0.
 //
 // Work item: route tile t (128 rows) x one 256-column block, one 256-thread
 // workgroup, two workgroups per CU.  Wave w owns all the rows and the columns
@@ -23,9 +23,16 @@
 // runs one (two) m tiles and stores the last computed row for the rest (37 tokens,
 // top-8, 39 tiles: 127 -> 94 us; 720 tokens, 56 tiles: 163 -> 131 us; the weights
 // alone stream in 65 / 95 us in that order of loads).  Its free registers hold weights
-// four steps ahead instead of two.  One-m-tile items load their weights
-// non-temporally (an expert with so few rows has one tile: 101 -> 94 us at 39 tiles);
-// two-m-tile items do not (152 against 147 us at 1500 tokens).
+// four steps ahead instead of two.
+//
+// Cache policy: up to 1.25 tiles per expert the weights are loaded non-temporally (one
+// tile reads them: 101 -> 94 us at 39 tiles, 143 -> 132 at 56, 184 -> 178 at 63); above,
+// full tiles share them through the L2s (548 tiles: 1174 against 1430 us non-temporal).
+//
+// Measured and not kept: the persistent form of these items (two workgroups per CU, the
+// next item's A stages and scales requested during the current one's last steps): fc1
+// 1412-1490 us, fc2 668 us over 548 tiles.  Its extra state spills at every item boundary,
+// and the second workgroup of the CU already covers an item's start.
 #pragma once
 
 #define K3B_STAGES 4
@@ -287,19 +294,73 @@ K3_DEV void k3b_run(const uint8_t* __restrict__ a, const uint8_t* __restrict__ a
   const int need = d1 ? 128 : d0 ? 65 - __builtin_clzll(d0) : 1;  // rows to compute
   v0 = v0 < 0 ? 0 : v0;
   v1 = v1 < 0 ? 0 : v1;
+  // About one tile per expert: no other tile reads these weights, and non-temporal loads
+  // stream them faster; with more, the L2s serve the second tile.
+  const int live = *num_tiles;
+  const bool once = live <= E + E / 4;
   if (need <= 32) {
     k3_v16f acc[1][2];
     k3b_loop<1, 4, 5, 8, true>(acc, a, a_sf, v0, v1, wb0, wb1, sbu, K, w, lane);
     epi(acc, std::integral_constant<int, 1>{}, tile, cb, e, w, lane);
   } else if (need <= 64) {
     k3_v16f acc[2][2];
-    k3b_loop<2, 4, 5, 8, false>(acc, a, a_sf, v0, v1, wb0, wb1, sbu, K, w, lane);
+    k3b_loop<2, 4, 5, 8, true>(acc, a, a_sf, v0, v1, wb0, wb1, sbu, K, w, lane);
     epi(acc, std::integral_constant<int, 2>{}, tile, cb, e, w, lane);
   } else {
     k3_v16f acc[4][2];
-    k3b_loop<4, 2, 3, 4, false>(acc, a, a_sf, v0, v1, wb0, wb1, sbu, K, w, lane);
+    if (once) k3b_loop<4, 2, 3, 4, true>(acc, a, a_sf, v0, v1, wb0, wb1, sbu, K, w, lane);
+    else k3b_loop<4, 2, 3, 4, false>(acc, a, a_sf, v0, v1, wb0, wb1, sbu, K, w, lane);
     epi(acc, std::integral_constant<int, 4>{}, tile, cb, e, w, lane);
   }
+}
+
+// bf16 out, stored as by k3w_gemm_bf16.
+K3_DEV void k3b_gemm_bf16(K3G_PARAMS, uint16_t* __restrict__ out) {
+  k3b_run(a, a_sf, a_rows, wt, wsf, num_tiles, cta_batch, E, N, K, max_tiles,
+          [&](auto& acc, auto mt_c, int tile, int cb, int, int w, int lane) {
+    constexpr int MT = decltype(mt_c)::value;
+    const int h = lane >> 5, j = lane & 31, p = lane & 1;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) {
+        uint32_t d[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) d[k] = k3_pack_bf2(acc[mt][nt][2 * k], acc[mt][nt][2 * k + 1]);
+        k3g_swap(d[0], d[4]);
+        k3g_swap(d[1], d[5]);
+        k3g_swap(d[2], d[6]);
+        k3g_swap(d[3], d[7]);
+        const k3_u4 X = {d[0], d[1], d[4], d[5]}, Y = {d[2], d[3], d[6], d[7]};
+        const k3_u4 snd = p ? X : Y;
+        k3_u4 rcv;
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          rcv[c] = (uint32_t)__builtin_amdgcn_mov_dpp((int)snd[c], K3_DPP_QP_1032, 0xf, 0xf, false);
+        const size_t row = (size_t)tile * K3G_TILE_M + 32 * mt + j;
+        uint16_t* o = out + (row & ~(size_t)1) * N + cb * K3G_TILE_N + 64 * w + 32 * nt +
+                      8 * (2 * h + p);
+        k3_st16(o, p ? rcv : X);
+        k3_st16(o + N, p ? Y : rcv);
+        if constexpr (MT < 4) {
+          if (mt == MT - 1) {  // rows past the computed ones: row 32 MT - 1's chunks
+            k3_u4 bx, by;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+              bx[c] = k3b_last(X[c], h);
+              by[c] = k3b_last(Y[c], h);
+            }
+#pragma unroll
+            for (int m = MT; m < 4; ++m) {
+              uint16_t* ob = out + ((size_t)tile * K3G_TILE_M + 32 * m + j) * N + cb * K3G_TILE_N +
+                             64 * w + 32 * nt + 16 * h;
+              k3_st16(ob, bx);
+              k3_st16(ob + 8, by);
+            }
+          }
+        }
+      }
+  });
 }
 
 K3_DEV void k3b_gemm_situ_mx(K3G_PARAMS, uint8_t* __restrict__ out_q, uint8_t* __restrict__ out_sf,
@@ -390,6 +451,10 @@ K3_DEV void k3b_gemm_acc(K3G_PARAMS, float* __restrict__ out) {
   extern "C" __global__ void __launch_bounds__(256, 2)                                           \
       kern_k3h_moe_gemm3_acc(K3G_PARAMS, float* __restrict__ out) {                              \
     k3b_gemm_acc(K3G_ARGS, out);                                                                 \
+  }                                                                                              \
+  extern "C" __global__ void __launch_bounds__(256, 2)                                           \
+      kern_k3h_moe_gemm3_bf16(K3G_PARAMS, uint16_t* __restrict__ out) {                          \
+    k3b_gemm_bf16(K3G_ARGS, out);                                                                \
   }                                                                                              \
   extern "C" __global__ void __launch_bounds__(256, 2)                                           \
       kern_k3h_moe_gemm3_situ_mx(K3G_PARAMS, uint8_t* __restrict__ out_q,                        \

@@ -329,3 +329,30 @@ def test_repeated_rows_match_gathered(ctx, K):
     for name, x, y in zip(("accumulators", "codes", "scales"), *got):
         bad = (x.reshape(nt, -1) != y.reshape(nt, -1)).any(1)
         assert not bad.any(), f"{name}: tiles {np.flatnonzero(bad)} differ"
+
+
+@pytest.mark.parametrize("N,K,gather", [(512, 512, False), (768, 3584, False), (3584, 768, True)])
+def test_bf16_few_tiles_match_many(ctx, N, K, gather):
+    """bf16 output on the register-weight items (max_tiles up to E + E / 16) against the
+    route for larger max_tiles over the same tiles, bit for bit, weights loaded
+    non-temporally (at most 1.25 E tiles); tiles past the live count, or whose expert is
+    out of range, keep their rows."""
+    E = 16
+    _case(f"bf16 few tiles E={E} N={N} K={K} gather={gather}")
+    few, many, nt = 17, 40, 15
+    g, q, sf, w, wsf = _inputs(8100 + N + K, many * 128, E, N, K)
+    cta = g.permutation(E)[:nt].astype(np.int32)
+    cta[3] = E
+    cta = np.concatenate([cta, np.zeros(many - nt, np.int32)])
+    rows = to_dev(g.integers(0, many * 128, many * 128).astype(np.int32)) if gather else None
+    wt, st = _tiled(ctx, w, wsf, E, N, K, 0)
+    da, dsf, dnt, dcta = to_dev(q), to_dev(sf), to_dev(np.array([nt], np.int32)), to_dev(cta)
+    outs = []
+    for max_tiles in (few, many):
+        o = torch.full((many * 128, N), 7.0, dtype=torch.bfloat16, device="cuda")
+        ctx.moe_gemm_mx(ctx.GEMM_BF16, da, dsf, rows, wt, st, dnt, dcta, max_tiles, E, N, K, o)
+        torch.cuda.synchronize()
+        outs.append(o)
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+    assert (outs[0][3 * 128:4 * 128] == 7).all() and (outs[0][nt * 128:] == 7).all()
+    assert not (outs[0][:3 * 128] == 7).all()
