@@ -8,7 +8,8 @@
 namespace {
 constexpr int kHeads = 24;
 constexpr int kInner = kHeads * 128;
-constexpr uint32_t kSpanShare = 2;  // 16-row tiles per span-gather workgroup
+constexpr uint32_t kSpanShare = 2;  // row tiles per span-gather workgroup
+constexpr int kSpanShort = 600;     // longest span of 4-row tiles (16-row ones above)
 }  // namespace
 
 extern "C" {
@@ -31,8 +32,12 @@ K3H_API int k3h_span_gather(k3h_ctx_t ctx, void* stream, const void* partial, co
   // taps pass through LDS): one work item per (tile pair, stream, column tile)
   // and one beta / flow item per tile pair, as a 1-D grid.  The entry also runs
   // the manifest's (INNER / 512, 4, ceil(span / 16)) x 128 geometry.
-  const uint32_t pairs = k3h_cdiv(k3h_cdiv(span, 16), kSpanShare);
-  return k3h_run(ctx, "k3_span_gather_v3+HEADS=24", "kern_k3_span_gather",
+  // Short spans take 4-row tiles: kernel time 16 rows 4.9 -> 3.3 us, 300 5.8 -> 5.0, 517
+  // 7.4 -> 7.1, 800 8.3 -> 9.9 (the re-read tap rows).
+  const bool is_short = span <= kSpanShort;
+  const uint32_t pairs = k3h_cdiv(k3h_cdiv(span, is_short ? 4 : 16), kSpanShare);
+  return k3h_run(ctx, "k3_span_gather_v3+HEADS=24",
+                 is_short ? "k3h_span_gather_short" : "kern_k3_span_gather",
                  (3 * (kInner / 512) + 1) * pairs, 1, 1, 128 * kSpanShare, stream, a);
 }
 

@@ -86,14 +86,18 @@ K3_DEV k3_u2 k9_ld8_nt(const uint16_t* p) { return __builtin_nontemporal_load((c
 
 #define K9_SHARE_MAX 4  // 16-row tiles per workgroup (block 128 x share)
 
-extern "C" __global__ void __launch_bounds__(128 * K9_SHARE_MAX) kern_k3_span_gather(
-    const uint16_t* __restrict__ partial, const float* __restrict__ cw, void* __restrict__ kda_base,
-    const int* __restrict__ line_index, long long line_bytes, const float* __restrict__ wsm_partial,
-    uint16_t* __restrict__ span_q, uint16_t* __restrict__ span_k, uint16_t* __restrict__ span_v,
-    uint16_t* __restrict__ span_beta, uint16_t* __restrict__ span_flow,
-    const int* __restrict__ span_at, int span) {
+#define K9_PARAMS                                                                             \
+  const uint16_t *__restrict__ partial, const float *__restrict__ cw,                        \
+      void *__restrict__ kda_base, const int *__restrict__ line_index, long long line_bytes, \
+      const float *__restrict__ wsm_partial, uint16_t *__restrict__ span_q,                  \
+      uint16_t *__restrict__ span_k, uint16_t *__restrict__ span_v,                          \
+      uint16_t *__restrict__ span_beta, uint16_t *__restrict__ span_flow,                    \
+      const int *__restrict__ span_at, int span
+
+template <int ROWS>
+K3_DEV void k9_span_gather(K9_PARAMS) {
   // A workgroup of 128 * share threads (share = blockDim.x / 128: 1 under the
-  // manifest's block, up to K9_SHARE_MAX) owns `share` consecutive 16-row tiles
+  // manifest's block, up to K9_SHARE_MAX) owns `share` consecutive ROWS-row tiles
   // of one column tile; thread group h (threads 128 h ..) owns tile h.  Tile h's
   // taps are tile h - 1's last three input rows, handed over through LDS, so the
   // workgroup reads the 3 rows before its first tile only.
@@ -104,7 +108,7 @@ extern "C" __global__ void __launch_bounds__(128 * K9_SHARE_MAX) kern_k3_span_ga
   // beta / flow groups, and the rest exit.  Every XCD then gets the same share.
   const int share = (int)blockDim.x / 128, half = (int)threadIdx.x / 128;
   const int tid = (int)threadIdx.x % 128;
-  const uint32_t nz = (uint32_t)(span + K9_ROWS - 1) / K9_ROWS;
+  const uint32_t nz = (uint32_t)(span + ROWS - 1) / ROWS;
   const uint32_t ng = (nz + share - 1) / share;
   const uint32_t L = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
   uint32_t bx, by, bg;
@@ -121,14 +125,14 @@ extern "C" __global__ void __launch_bounds__(128 * K9_SHARE_MAX) kern_k3_span_ga
   }
   const uint32_t bz = bg * share + half;
   const int at = span_at[0];
-  const int tile0 = bz * K9_ROWS;
+  const int tile0 = bz * ROWS;
   partial += (size_t)at * K9_KDA_FUSED;
   wsm_partial += (size_t)at * K9_WSM;
 
   if (by == 3) {
     // 8 threads per row: thread k lands beta for heads k, k + 8, ... and 16 flow columns
     const int i = tile0 + tid / 8, k = tid % 8;
-    if (i >= span) return;
+    if (tid / 8 >= ROWS || i >= span) return;
     const float* row = wsm_partial + (size_t)i * K9_WSM;
     for (int h = k; h < HEADS; h += 8) span_beta[(size_t)h * span + i] = (uint16_t)k3_pack_bf2(row[h], 0.0f);
     const float4* fa = (const float4*)(row + K9_WSM_FA + k * 16);
@@ -148,7 +152,7 @@ extern "C" __global__ void __launch_bounds__(128 * K9_SHARE_MAX) kern_k3_span_ga
   const int row0 = tile0;
   // rows of this tile; 0 for a thread group past the span's last tile (it loads
   // and stores nothing but still meets the workgroup barrier)
-  const int nrow = max(0, min(K9_ROWS, span - row0));
+  const int nrow = max(0, min(ROWS, span - row0));
   uint16_t* __restrict__ out = s == 0 ? span_q : s == 1 ? span_k : span_v;
   const uint16_t* __restrict__ col = partial + (size_t)s * K9_INNER + c;
   const bool first = bz == 0;
@@ -164,7 +168,7 @@ extern "C" __global__ void __launch_bounds__(128 * K9_SHARE_MAX) kern_k3_span_ga
     for (int k = 0; k < 4; ++k) w[t][k] = __uint_as_float(a[k]);
   }
   // x[j] = input row row0 - 3 + j (j < 3: taps)
-  k3_u2 x[K9_ROWS + 3];
+  k3_u2 x[ROWS + 3];
   if (half == 0) {
 #pragma unroll
     for (int t = 0; t < 3; ++t)
@@ -173,14 +177,14 @@ extern "C" __global__ void __launch_bounds__(128 * K9_SHARE_MAX) kern_k3_span_ga
   }
   if (nrow > 0) {
 #pragma unroll
-    for (int r = 0; r < K9_ROWS; ++r)
+    for (int r = 0; r < ROWS; ++r)
       x[3 + r] = k9_ld8_nt(col + (size_t)(row0 + min(r, nrow - 1)) * K9_KDA_FUSED);
   }
   if (share > 1) {
     __shared__ k3_u2 taps_s[K9_SHARE_MAX - 1][3][128];
     if (half < share - 1 && nrow > 0) {
 #pragma unroll
-      for (int t = 0; t < 3; ++t) taps_s[half][t][tid] = x[K9_ROWS + t];
+      for (int t = 0; t < 3; ++t) taps_s[half][t][tid] = x[ROWS + t];
     }
     __syncthreads();
     if (half > 0) {
@@ -196,7 +200,7 @@ extern "C" __global__ void __launch_bounds__(128 * K9_SHARE_MAX) kern_k3_span_ga
   k9_unpack4(x[1], a[1]);
   k9_unpack4(x[2], a[2]);
 #pragma unroll
-  for (int r = 0; r < K9_ROWS; ++r) {
+  for (int r = 0; r < ROWS; ++r) {
     k9_unpack4(x[3 + r], a[(r + 3) & 3]);
     const k3_u2 o = k9_row(a[r & 3], a[(r + 1) & 3], a[(r + 2) & 3], a[(r + 3) & 3], w);
     if (r < nrow) __builtin_nontemporal_store(o, (k3_u2*)(out + (size_t)(row0 + r) * K9_INNER + c));
@@ -214,4 +218,18 @@ extern "C" __global__ void __launch_bounds__(128 * K9_SHARE_MAX) kern_k3_span_ga
 #pragma unroll
     for (int t = 0; t < 3; ++t) *(k3_u2*)(win + (size_t)t * K9_INNER + c) = nt[t];
   }
+}
+
+extern "C" __global__ void __launch_bounds__(128 * K9_SHARE_MAX) kern_k3_span_gather(K9_PARAMS) {
+  k9_span_gather<K9_ROWS>(partial, cw, kda_base, line_index, line_bytes, wsm_partial, span_q, span_k,
+                          span_v, span_beta, span_flow, span_at, span);
+}
+
+// Short spans: 4-row tiles.  With 16 a span of a few hundred rows has fewer waves than the
+// chip has SIMDs, and each of them evaluates 64 activations one after another; the tap
+// rows that shorter tiles read again come from the L2s (kernel time 16 rows 4.9 -> 3.3 us,
+// 300 5.8 -> 5.0, 517 7.4 -> 7.1, 800 8.3 -> 9.9: the typed call takes it up to 600 rows).
+extern "C" __global__ void __launch_bounds__(128 * K9_SHARE_MAX) k3h_span_gather_short(K9_PARAMS) {
+  k9_span_gather<4>(partial, cw, kda_base, line_index, line_bytes, wsm_partial, span_q, span_k,
+                    span_v, span_beta, span_flow, span_at, span);
 }

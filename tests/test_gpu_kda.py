@@ -260,3 +260,11 @@ def test_kda_out_gate_special_values(ctx):
     torch.cuda.synchronize()
     got = from_dev(gated)
     _special_match("gated", got[at:at + span], want[at:at + span])
+
+
+@pytest.mark.parametrize("span", [1, 2, 3, 4, 5, 8, 9, 599, 600, 601])
+def test_span_gather_short_matches_manifest(ctx, span):
+    """The typed call's 4-row tiles (spans up to 600) against the manifest geometry, bit
+    for bit: spans under the window, partial tiles, a pair whose second tile is empty,
+    both sides of the longest short span."""
+    test_span_gather_manifest_geometry_matches_typed(ctx, span)
