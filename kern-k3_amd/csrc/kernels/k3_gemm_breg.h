@@ -23,7 +23,14 @@
 // runs one (two) m tiles and stores the last computed row for the rest (37 tokens,
 // top-8, 39 tiles: 127 -> 94 us; 720 tokens, 56 tiles: 163 -> 131 us; the weights
 // alone stream in 65 / 95 us in that order of loads).  Its free registers hold weights
-// four steps ahead instead of two.
+// six steps ahead instead of two, and its free LDS the A rows eight (six) steps ahead
+// (39 tiles 95.6 us at four / five steps, 92.2 at six; 56 tiles 133.4 -> 127.5; eight
+// steps no faster).
+//
+// Without a row list (fc2) every row is computed.  There the A rows, not their MFMAs, are
+// the cost: 16 KB per step and workgroup, as many bytes as the weights.  Finding the
+// repeated rows by comparing them on the way reads them all the same and gains nothing
+// (39 tiles 71.9 against 72.0 us; with the rows known it would be 60).
 //
 // Cache policy: up to 1.25 tiles per expert the weights are loaded non-temporally (one
 // tile reads them: 101 -> 94 us at 39 tiles, 143 -> 132 at 56, 184 -> 178 at 63); above,
@@ -68,6 +75,15 @@ K3_DEV uint32_t k3b_last(uint32_t v, int h) {
   return h ? hi : lo;
 }
 
+// f(0), f(1), .. f(N - 1), the index a compile-time constant.
+template <int N, int I = 0, class F>
+K3_DEV void k3b_each(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    k3b_each<N, I + 1>(f);
+  }
+}
+
 // The K loop of one item over the tile's first 32 MT rows, for the wave's 64 columns.
 // NB: weight buffers (a step's weights are requested NB steps ahead); PA: stages the A
 // rows are requested ahead (ring of RS stages); NTW: weights loaded non-temporally.
@@ -80,6 +96,8 @@ K3_DEV void k3b_loop(k3_v16f (&acc)[MT][2], const uint8_t* __restrict__ a,
   constexpr int P = 5 + MT;       // vector-memory operations a wave issues per step
   constexpr int LK = MT < 2 ? 1 : 2;  // units the A operands are read ahead
   static_assert(RS * STG <= K3B_SAT_OFF && (RS & (RS - 1)) == 0 && RS > PA, "A ring");
+  static_assert(2 * MT * NB % 4 == 0, "the A operand buffers' turn");
+  static_assert(NB * P < 64, "the vector-memory counter");
   const int h = lane >> 5, j = lane & 31;
   const int KG = K / 32, KS = K / K3G_KSTEP;
   uint8_t* lds = k3b_smem();
@@ -108,14 +126,11 @@ K3_DEV void k3b_loop(k3_v16f (&acc)[MT][2], const uint8_t* __restrict__ a,
   };
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
-  using I2 = std::integral_constant<int, 2>;
-  using I3 = std::integral_constant<int, 3>;
-  load_b(I0{}, I0{}, 0); load_b(I0{}, I1{}, 0); sb[0] = load_sb(0);
-  load_b(I1{}, I0{}, 1); load_b(I1{}, I1{}, 1); sb[1] = load_sb(1);
-  if constexpr (NB > 2) {
-    load_b(I2{}, I0{}, 2); load_b(I2{}, I1{}, 2); sb[2] = load_sb(2);
-    load_b(I3{}, I0{}, 3); load_b(I3{}, I1{}, 3); sb[3] = load_sb(3);
-  }
+  k3b_each<NB>([&](auto i) {
+    load_b(i, I0{}, i);
+    load_b(i, I1{}, i);
+    sb[i] = load_sb(i);
+  });
   K3B_FENCE();
   // this wave's A loads: row slices 8 q .. + 8, q = MT w + b
   uint32_t arow[MT];
@@ -137,14 +152,27 @@ K3_DEV void k3b_loop(k3_v16f (&acc)[MT][2], const uint8_t* __restrict__ a,
 #pragma unroll
   for (int k = 0; k < PA; ++k) issue_a(k);
   {
-    constexpr int TPR = 8 / MT;  // threads per A-scale row
+    // All of a row's scales in flight at once, C dwords per thread.  A row that fills the
+    // table (K = 3584) gives each thread C consecutive ones, in wide loads (548 tiles 1164
+    // us, dword by dword 1167-1183); a shorter one repeats its last (K = 3072: 67 us over
+    // 39 tiles, 69 with a loop over the dwords).
+    constexpr int TPR = 8 / MT, C = (K3B_KGM / 4 + TPR - 1) / TPR;  // threads per A-scale row
     const int row = threadIdx.x / TPR, part = threadIdx.x % TPR, KGd = KG / 4;
-    const int d0 = KGd * part / TPR, d1 = KGd * (part + 1) / TPR;
     const uint32_t src = (uint32_t)__shfl(MT < 4 || w < 2 ? v0 : v1, row & 63, 64);
     const uint32_t* sr = (const uint32_t*)(a_sf + (size_t)src * KG);
     uint32_t* dr = (uint32_t*)(sat + row * K3G_SAT_ROW(K3B_KGM));
-#pragma unroll 14
-    for (int d = d0; d < d1; ++d) dr[d] = sr[d];
+    uint32_t x[C];
+    if (KGd == TPR * C) {
+#pragma unroll
+      for (int c = 0; c < C; ++c) x[c] = sr[C * part + c];
+#pragma unroll
+      for (int c = 0; c < C; ++c) dr[C * part + c] = x[c];
+    } else {
+#pragma unroll
+      for (int c = 0; c < C; ++c) x[c] = sr[min(part + TPR * c, KGd - 1)];
+#pragma unroll
+      for (int c = 0; c < C; ++c) dr[min(part + TPR * c, KGd - 1)] = x[c];
+    }
   }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
@@ -246,20 +274,11 @@ K3_DEV void k3b_loop(k3_v16f (&acc)[MT][2], const uint8_t* __restrict__ a,
     K3B_FENCE();
   };
   int ks = 0;  // KS is even
-  for (; ks + NB <= KS; ks += NB) {
-    step(ks, I0{});
-    step(ks + 1, I1{});
-    if constexpr (NB > 2) {
-      step(ks + 2, I2{});
-      step(ks + 3, I3{});
-    }
-  }
-  if constexpr (NB > 2) {
-    if (ks < KS) {
-      step(ks, I0{});
-      step(ks + 1, I1{});
-    }
-  }
+  for (; ks + NB <= KS; ks += NB) k3b_each<NB>([&](auto i) { step(ks + i, i); });
+  if constexpr (NB > 2)  // the last KS % NB
+    k3b_each<NB - 1>([&](auto i) {
+      if (ks + i < KS) step(ks + i, i);
+    });
   __builtin_amdgcn_s_waitcnt(0);  // no load into LDS outlives the workgroup
 }
 
@@ -300,11 +319,11 @@ K3_DEV void k3b_run(const uint8_t* __restrict__ a, const uint8_t* __restrict__ a
   const bool once = live <= E + E / 4;
   if (need <= 32) {
     k3_v16f acc[1][2];
-    k3b_loop<1, 4, 5, 8, true>(acc, a, a_sf, v0, v1, wb0, wb1, sbu, K, w, lane);
+    k3b_loop<1, 6, 8, 16, true>(acc, a, a_sf, v0, v1, wb0, wb1, sbu, K, w, lane);
     epi(acc, std::integral_constant<int, 1>{}, tile, cb, e, w, lane);
   } else if (need <= 64) {
     k3_v16f acc[2][2];
-    k3b_loop<2, 4, 5, 8, true>(acc, a, a_sf, v0, v1, wb0, wb1, sbu, K, w, lane);
+    k3b_loop<2, 6, 6, 8, true>(acc, a, a_sf, v0, v1, wb0, wb1, sbu, K, w, lane);
     epi(acc, std::integral_constant<int, 2>{}, tile, cb, e, w, lane);
   } else {
     k3_v16f acc[4][2];

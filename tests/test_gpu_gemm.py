@@ -291,7 +291,7 @@ def test_wide_items_match_4wave(ctx, K):
             assert same
 
 
-@pytest.mark.parametrize("K", [512, 768, 3584])
+@pytest.mark.parametrize("K", [512, 768, 1024, 3584])
 def test_repeated_rows_match_gathered(ctx, K):
     """Tiles padded by repeating a row index (the fc1 kernel computes one or two m tiles
     and repeats the last row's results) against the same rows gathered beforehand
