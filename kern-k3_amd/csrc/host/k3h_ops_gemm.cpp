@@ -149,8 +149,8 @@ K3H_API int k3h_moe_gemm_mx(k3h_ctx_t ctx, void* stream, int epilogue, const voi
   const uint32_t rows = gemm_grid_rows(max_tiles, N / kTileN);
   // bf16 with hardly a row per expert (max_tiles counts a partial tile for each): the
   // weights' stream bounds it, and 256-column items on two workgroups per CU stream them
-  // faster as long as they fit about one round (1 tile 29 -> 22 us, 39 tiles 86 -> 71, but 56
-  // tiles 93 -> 98)
+  // faster as long as they fit about one round (1 tile 29 -> 22 us, 39 tiles 86 -> 68, but 56
+  // tiles 93 -> 96)
   if (epilogue == K3H_GEMM_BF16 && breg && max_tiles <= E + E / 16 && rows <= 65535u)
     return k3h_run(ctx, "k3h_moe_gemm", "kern_k3h_moe_gemm3_bf16", (uint32_t)(N / kTileN), rows, 1,
                    kBlock, stream, args);

@@ -21,10 +21,10 @@
 // routing tables pad a tile by repeating a row index, so every row past the last
 // distinct index has the last one's results: a tile that needs at most 32 (64) rows
 // runs one (two) m tiles and stores the last computed row for the rest (37 tokens,
-// top-8, 39 tiles: 127 -> 94 us; 720 tokens, 56 tiles: 163 -> 131 us; the weights
+// top-8, 39 tiles: 127 -> 91 us; 720 tokens, 56 tiles: 163 -> 127 us; the weights
 // alone stream in 65 / 95 us in that order of loads).  Its free registers hold weights
 // six steps ahead instead of two, and its free LDS the A rows eight (six) steps ahead
-// (39 tiles 95.6 us at four / five steps, 92.2 at six; 56 tiles 133.4 -> 127.5; eight
+// (39 tiles 95.6 us at four / five steps, 91.2 at six; 56 tiles 133.4 -> 127; eight
 // steps no faster).
 //
 // Without a row list (fc2) every row is computed.  There the A rows, not their MFMAs, are

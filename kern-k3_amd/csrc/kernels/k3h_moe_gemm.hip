@@ -19,6 +19,9 @@
 //        u = bf16(C[r, j]), g = bf16(C[r, N / 2 + j]) the activation
 //        x = bf16(situ(g, u; alpha[e], beta[e])) is quantised per 32 columns
 //        exactly as kern_k3_moe_quant quantises a bf16 row)
+// These take every K; 512 <= K <= 3584, K % 256 == 0 runs the register-weight items of
+// k3_gemm_breg.h for fc1 and for fc2 over few tiles, and 512-column blocks the persistent
+// items of k3_gemm_wide.h for the other f32 / bf16 products, the same products bit for bit.
 //
 // Weight layouts (built once at load time by kern_k3h_moe_w_tile /
 // kern_k3h_moe_sf_tile from the row-major [E, N, K / 2] e2m1 (low nibble = even
