@@ -98,6 +98,7 @@ K3_DEV void k3b_loop(k3_v16f (&acc)[MT][2], const uint8_t* __restrict__ a,
   static_assert(RS * STG <= K3B_SAT_OFF && (RS & (RS - 1)) == 0 && RS > PA, "A ring");
   static_assert(2 * MT * NB % 4 == 0, "the A operand buffers' turn");
   static_assert(NB * P < 64, "the vector-memory counter");
+  static_assert(PA + 1 >= NB, "every A stage is requested before the last KS % NB steps");
   const int h = lane >> 5, j = lane & 31;
   const int KG = K / 32, KS = K / K3G_KSTEP;
   uint8_t* lds = k3b_smem();
@@ -105,8 +106,9 @@ K3_DEV void k3b_loop(k3_v16f (&acc)[MT][2], const uint8_t* __restrict__ a,
   uint32_t lo16 = 16u * (uint32_t)lane, lo8 = 8u * (uint32_t)lane;
 
   // scalar-base loads: the step's wave-uniform address is held in scalar registers and
-  // the lane's offset added last; requests past the last step repeat it (their data is
-  // not used), so that every step issues the same operations
+  // the lane's offset added last; requests past the last step repeat it, so that every
+  // step of the counted loop issues the same operations (the use after the loop keeps
+  // those whose data no step reads)
   k3_u4 bv[NB][2][2];  // [buffer][substep][n tile]
   uint32_t sb[NB];
   auto load_b = [&](auto bi_c, auto s_c, int k) {
@@ -214,9 +216,11 @@ K3_DEV void k3b_loop(k3_v16f (&acc)[MT][2], const uint8_t* __restrict__ a,
 #pragma unroll
       for (int nt = 0; nt < 2; ++nt) asm volatile("" : "+v"(acc[mt][nt]));
   };
-  // One K step with weights in buffer BI.
-  auto step = [&](int ks, auto bi_c) {
+  // One K step with weights in buffer BI.  TAIL: everything it reads has landed and no
+  // later step needs more, so it requests nothing and waits for nothing.
+  auto step = [&](int ks, auto bi_c, auto tail_c) {
     constexpr int BI = decltype(bi_c)::value;
+    constexpr bool TAIL = decltype(tail_c)::value;
 #pragma unroll
     for (int b = 0; b < MT; ++b) asm volatile("" : "+v"(arow[b]));
     asm volatile("" : "+v"(lo16), "+v"(lo8));
@@ -247,20 +251,22 @@ K3_DEV void k3b_loop(k3_v16f (&acc)[MT][2], const uint8_t* __restrict__ a,
     };
     // the step's first weights and scales have landed (left to itself the compiler
     // would wait here for every load in flight)
-    __builtin_amdgcn_s_waitcnt(K3W_VMCNT(2 + (NB - 1) * P));
+    if constexpr (!TAIL) __builtin_amdgcn_s_waitcnt(K3W_VMCNT(2 + (NB - 1) * P));
     half(I0{});
     uint32_t san[MT];
     pin();
     K3B_FENCE();
-    load_b(bi_c, I0{}, ks + NB);
-    K3B_FENCE();
-    // this step's second weights and the A rows of step ks + 1 have landed
-    constexpr int WB = 2 + (NB - 1) * P, WA = 5 + (PA - 2) * P;
-    __builtin_amdgcn_s_waitcnt(K3W_VMCNT(WA < WB ? WA : WB));
-    __builtin_amdgcn_s_barrier();
-    K3B_FENCE();
-    issue_a(ks + PA);
-    K3B_FENCE();
+    if constexpr (!TAIL) {
+      load_b(bi_c, I0{}, ks + NB);
+      K3B_FENCE();
+      // this step's second weights and the A rows of step ks + 1 have landed
+      constexpr int WB = 2 + (NB - 1) * P, WA = 5 + (PA - 2) * P;
+      __builtin_amdgcn_s_waitcnt(K3W_VMCNT(WA < WB ? WA : WB));
+      __builtin_amdgcn_s_barrier();
+      K3B_FENCE();
+      issue_a(ks + PA);
+      K3B_FENCE();
+    }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) san[mt] = rd_sa(ks + 1, mt);
     half(I1{});
@@ -268,18 +274,32 @@ K3_DEV void k3b_loop(k3_v16f (&acc)[MT][2], const uint8_t* __restrict__ a,
     for (int mt = 0; mt < MT; ++mt) sa[mt] = san[mt];
     pin();
     K3B_FENCE();
-    sb[BI] = load_sb(ks + NB);
-    K3B_FENCE();
-    load_b(bi_c, I1{}, ks + NB);
-    K3B_FENCE();
+    if constexpr (!TAIL) {
+      sb[BI] = load_sb(ks + NB);
+      K3B_FENCE();
+      load_b(bi_c, I1{}, ks + NB);
+      K3B_FENCE();
+    }
   };
   int ks = 0;  // KS is even
-  for (; ks + NB <= KS; ks += NB) k3b_each<NB>([&](auto i) { step(ks + i, i); });
-  if constexpr (NB > 2)  // the last KS % NB
-    k3b_each<NB - 1>([&](auto i) {
-      if (ks + i < KS) step(ks + i, i);
-    });
+  for (; ks + NB <= KS; ks += NB)
+    k3b_each<NB>([&](auto i) { step(ks + i, i, std::false_type{}); });
+  K3B_FENCE();
   __builtin_amdgcn_s_waitcnt(0);  // no load into LDS outlives the workgroup
+  if constexpr (NB > 2) {         // the last KS % NB: every wave's requests have landed
+    if (ks < KS) {
+      __builtin_amdgcn_s_barrier();
+      K3B_FENCE();
+      k3b_each<NB - 1>([&](auto i) {
+        if (ks + i < KS) step(ks + i, i, std::true_type{});
+      });
+    }
+  }
+  // the counted waits of the last turn include loads past the last step: they stay
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+    asm volatile("" ::"v"(bv[i][0][0]), "v"(bv[i][0][1]), "v"(bv[i][1][0]), "v"(bv[i][1][1]),
+                 "v"(sb[i]));
 }
 
 template <class Epi>
