@@ -7,10 +7,15 @@ const char* quant_key(int v2) { return v2 ? "k3_quant_fp8_pair_v2" : "k3_quant_f
 // k3h_quant_fp8_once (one launch that keeps most of x on the chip between the passes): one
 // workgroup per CU, the manifest's nb only.
 constexpr int kOnceNb = 2048, kOnceGrid = 256, kOnceBlock = 1024;
-// below, its fixed cost exceeds the second read of x (20.9 -> 18.4 us at n = 25 M, 15.2 ->
-// 16.7 us at 18 M)
+// below, its fixed cost exceeds the second read of x (back to back over three sets 20.8 ->
+// 18.7 us at n = 25 M, 18.0 -> 17.8 at 21 M)
 constexpr int kOnceMinN = 24 << 20;
-constexpr int kOnceSpinTicks = 20000;  // 200 us of the 100 MHz clock
+// How long a workgroup waits for the others' partials before it takes the missing ones
+// itself, in ticks of the 100 MHz clock: twice the undisturbed meeting (4 us), and an eighth
+// of the reading time, by which the workgroups' ends differ (at n = 537 M 414 us; 450 with 8
+// us for every n).  Longer only costs the call whose workgroups are kept out (beside a
+// one-wave kernel at n = 25 M: 54 us at 8 us, 77 at 30).
+int once_spin_ticks(int n) { return 800 + (n >> 18); }
 bool quant_args_ok(const void* x, int n, const void* partials, int nb) {
   return n >= 0 && nb >= 1 && nb <= 65535 && k3h_okp(x, 16) && k3h_okp(partials, 4);
 }
@@ -53,7 +58,7 @@ K3H_API int k3h_quant_fp8_tensor(k3h_ctx_t ctx, void* stream, int v2, const void
                             kOnceBlock, stream, m);
       if (r != K3H_OK) return r;
       K3hArgs a;
-      a.ptr(x).ptr(y).i32(n).ptr(partials).ptr(scale_out).i32(kOnceSpinTicks);
+      a.ptr(x).ptr(y).i32(n).ptr(partials).ptr(scale_out).i32(once_spin_ticks(n));
       return k3h_run(ctx, quant_key(1), "k3h_quant_fp8_once", kOnceGrid, 1, 1, kOnceBlock, stream, a);
     }
   }

@@ -143,15 +143,19 @@ extern "C" __global__ void __launch_bounds__(QT) K3_APPLY_NAME(
 // the outputs of the pair at nb = 2048 bit for bit (partials included).  The pair reads
 // x twice, and although the second pass comes from the MALL it costs as much as the
 // first.  Here one persistent launch (256 workgroups of 1024 threads, one per CU) keeps
-// the last 24 of a thread's vectors on the chip (15 in registers, 9 in LDS: 98 MB of
+// the last 24 of a thread's vectors on the chip (15 in registers, 9 in LDS: 100.7 MB of
 // x in all), meets at the partials, and quantises what it holds; only the vectors before
 // those are read again, from the MALL.  Quarter s of workgroup g plays the pair's blocks
 // 8 g + s and 8 g + 4 + s, so a thread's m-th vector is vector
 // (8 g + 4 (m & 1) + s + 2048 (m >> 1)) * 256 + t and the chip sweeps x front to back.
-// Measured over three rotating sets: n = 117 M 87.2 -> 74.8 us, 59 M 44.9 -> 33.7, 29 M
-// 23.9 -> 19.5, 25 M 20.9 -> 18.4, 18 M 15.2 -> 16.7 (mark, dispatch and the meeting cost
+// Measured over three rotating sets: n = 117 M 87.2 -> 74.8 us, 59 M 44.9 -> 33.7, 34 M
+// 26.5 -> 21.2, 25 M 20.8 -> 18.7, 21 M 18.0 -> 17.8 (mark, dispatch and the meeting cost
 // about 13 us): the host takes it for n >= 24 << 20.  At 117 M a workgroup spends 36 us
 // reading (6.5 TB/s), 4 us meeting and 20 us on the second pass.
+// A workgroup fills its CU, so another stream's kernel on one CU (one wave will do) keeps
+// one of the 256 out until the others end: n = 117 M beside such a wave 120 us (the pair 97),
+// 25 M 55 us (25); beside a large copy or GEMM both streams together take as long as with
+// the pair.
 // Requires n >= 8.
 #define QO_NB 2048
 #define QO_REG 15           // vectors a thread keeps in registers
@@ -289,13 +293,17 @@ extern "C" __global__ void __launch_bounds__(1024) k3h_quant_fp8_once(
 #pragma unroll
     for (int k = 0; k < 4; ++k) v[0][k] = __builtin_nontemporal_load(at(again(k)));
   }
-  // every block's partial: poll until it is set, for spin_ticks (10 ns each) at most
+  // every block's partial (slots tid and 1024 + tid): poll until it is set, for spin_ticks
+  // (10 ns each) at most
+  auto poll = [&](int slot) -> uint32_t {
+    return __hip_atomic_load(partials + slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
   uint32_t p0, p1;
   {
     const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
     for (;;) {
-      p0 = __hip_atomic_load(partials + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      p1 = __hip_atomic_load(partials + 1024 + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      p0 = poll(tid);
+      p1 = poll(1024 + tid);
       if (__ballot(p0 == QO_UNSET || p1 == QO_UNSET) == 0) break;
       if ((uint64_t)__builtin_amdgcn_s_memrealtime() - t0 >= (uint64_t)spin_ticks) break;
       __builtin_amdgcn_s_sleep(1);
@@ -304,56 +312,80 @@ extern "C" __global__ void __launch_bounds__(1024) k3h_quant_fp8_once(
   // the max over the partials that are not NaN patterns (those compare as bits in
   // `partials`, and the scale ignores them)
   auto fold = [&](float f, uint32_t p) { return p == QO_UNSET ? f : __builtin_fmaxf(f, __uint_as_float(p)); };
-  float amax = fold(fold(0.0f, p0), p1);
   __shared__ float fred[16];
-  __shared__ int missing[16];
-  {
+  __shared__ int short_of[16];
+  auto wave_fold = [&]() {
+    float f = fold(fold(0.0f, p0), p1);
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) amax = __builtin_fmaxf(amax, __shfl_xor(amax, o, 64));
+    for (int o = 32; o > 0; o >>= 1) f = __builtin_fmaxf(f, __shfl_xor(f, o, 64));
+    if ((tid & 63) == 0) fred[wave] = f;
+  };
+  wave_fold();
+  {
     const bool miss = __ballot(p0 == QO_UNSET || p1 == QO_UNSET) != 0;
-    if ((tid & 63) == 0) {
-      fred[wave] = amax;
-      missing[wave] = miss;
-    }
+    if ((tid & 63) == 0) short_of[wave] = miss;
   }
   __syncthreads();
+  float amax = 0.0f;
   bool any = false;
 #pragma unroll
   for (int k = 0; k < 16; ++k) {
     amax = __builtin_fmaxf(amax, fred[k]);
-    any |= missing[k] != 0;
+    any |= short_of[k] != 0;
   }
   if (any) {
-    // A workgroup that is not resident yet cannot have set its partials (the device is
-    // shared): the waiting ones take the missing blocks' maxima themselves, each starting
-    // at another block and storing what it finds for the others, so no workgroup ever
-    // depends on another one running.
-    for (int c = 0; c < QO_NB; ++c) {
-      const int b = (c + 8 * (int)blockIdx.x) & (QO_NB - 1);
-      __syncthreads();
-      if (tid == 0)
-        red[1][0] = __hip_atomic_load(partials + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __syncthreads();
-      uint32_t p = red[1][0];  // the same for the whole workgroup
-      if (p == QO_UNSET) {
-        uint32_t bm = 0;
-        for (long long i = (b + (long long)QO_NB * s) * 256 + t; i < nv; i += 4LL * QO_NB * 256)
-          bm = k3_qo_max(bm, k3_ld16(x + i * 8));
-        if (b == 0 && tid < (n & 7)) {
-          const uint32_t a = x[nv * 8 + tid] & 0x7fffu;
-          bm = bm > a ? bm : a;
-        }
-        bm = k3_qo_wave_max(bm);
-        if ((tid & 63) == 0) red[0][wave] = bm;
-        __syncthreads();
-#pragma unroll
-        for (int v = 0; v < 16; ++v) bm = bm > red[0][v] ? bm : red[0][v];
-        p = bm << 16;
-        if (tid == 0)
-          __hip_atomic_store(partials + b, p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    // A workgroup that is not resident yet cannot have set its partials (another stream's
+    // kernel holds its CU): the waiting ones take the missing blocks' maxima themselves, one
+    // block a turn, spread over the missing ones by workgroup, storing what they find for
+    // the others and looking again what those have found.  No workgroup ever depends on
+    // another one running, and a turn sets at least one of its partials, so this ends.
+    __shared__ uint64_t missing[32];  // bit i of [k]: block 64 k + i
+    for (;;) {
+      const uint64_t m0 = __ballot(p0 == QO_UNSET), m1 = __ballot(p1 == QO_UNSET);
+      if ((tid & 63) == 0) {
+        missing[wave] = m0;
+        missing[16 + wave] = m1;
       }
-      amax = __builtin_fmaxf(amax, __uint_as_float(p));
+      __syncthreads();
+      uint32_t left = 0;
+      for (int k = 0; k < 32; ++k) left += (uint32_t)__popcll(missing[k]);
+      if (left == 0) break;
+      // the workgroup's pick among the `left` missing blocks, the same in every thread
+      uint32_t pick = (blockIdx.x * left) / gridDim.x;
+      int b = 0;
+      for (int k = 0; k < 32; ++k) {
+        uint64_t m = missing[k];
+        const uint32_t c = (uint32_t)__popcll(m);
+        if (pick < c) {
+          for (; pick > 0; --pick) m &= m - 1;
+          b = 64 * k + __builtin_ctzll(m);
+          break;
+        }
+        pick -= c;
+      }
+      uint32_t bm = 0;
+#pragma unroll 1
+      for (uint32_t i = (uint32_t)(b + QO_NB * s) * 256u + (uint32_t)t; i <= last; i += 4u * QO_NB * 256u)
+        bm = k3_qo_max(bm, *at(i));
+      if (b == 0 && tid < (n & 7)) {
+        const uint32_t a = x[nv * 8 + tid] & 0x7fffu;
+        bm = bm > a ? bm : a;
+      }
+      bm = k3_qo_wave_max(bm);
+      if ((tid & 63) == 0) red[0][wave] = bm;
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < 16; ++k) bm = bm > red[0][k] ? bm : red[0][k];
+      const uint32_t p = bm << 16;
+      if (tid == 0)
+        __hip_atomic_store(partials + b, p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      if (p0 == QO_UNSET) p0 = b == tid ? p : poll(tid);
+      if (p1 == QO_UNSET) p1 = b == 1024 + tid ? p : poll(1024 + tid);
     }
+    wave_fold();
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 16; ++k) amax = __builtin_fmaxf(amax, fred[k]);
   }
   const float scale = amax > 0.0f ? amax / 448.0f : 1.0f;
   if (blockIdx.x == 0 && tid == 0 && scale_out) *scale_out = scale;

@@ -148,3 +148,87 @@ def test_quant_fp8_tensor_route(ctx, n):
     torch.cuda.synchronize()
     assert np.array_equal(from_dev(p), want_p) and from_dev(s)[0] == want_s[0]
     assert np.array_equal(from_dev(y)[:n], want_y)
+
+
+@pytest.mark.parametrize("n", [24 << 20, (15 << 22) + 4099])
+def test_quant_fp8_tensor_beside_a_waiting_wave(ctx, n):
+    """The one-launch form while one wave of another stream (the arrival wait for a rank that
+    never arrives, 20 ms) holds a CU, so that one of its workgroups starts only after others
+    have ended: the pair's outputs, and no long wait.  The bound is the 200 us that a
+    workgroup would once have waited before it took the missing maxima itself (measured:
+    713-770 us then; 55 us at 25 M, 75 us at 63 M now)."""
+    print(f"[case] quant_fp8_tensor beside a waiting wave n={n}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(1500 + n % 97)
+    x = torch.empty(n, device="cuda").normal_(0, 2, generator=g).to(torch.bfloat16)
+    nb = 2048
+    y, want_y = (torch.full((n + 8,), 0x5a, dtype=torch.uint8, device="cuda") for _ in range(2))
+    s, want_s = (torch.zeros(1, dtype=torch.float32, device="cuda") for _ in range(2))
+    p, want_p = (torch.empty(nb, dtype=torch.float32, device="cuda") for _ in range(2))
+    stream = torch.cuda.current_stream().cuda_stream
+    assert ctx.L.k3h_quant_fp8_amax(ctx.h, stream, 1, x.data_ptr(), n, want_p.data_ptr(), nb) == 0
+    assert ctx.L.k3h_quant_fp8_apply(ctx.h, stream, 1, x.data_ptr(), want_y.data_ptr(), n,
+                                     want_p.data_ptr(), nb, want_s.data_ptr()) == 0
+    arrive = k3h.ManifestOp(ctx, "arrive", {
+        "params": ["out buffer<u64>", "in buffer<u64>", "i32", "i32", "i32", "out buffer<u32>"],
+        "impl": {"launches": [{"module": "k3_rs_arrive_v2+K3_SPIN_US=20000",
+                               "entry": "k3h_rs_arrive_mask", "block": [64, 1, 1], "grid": [1, 1, 1]}]}})
+    own, peer = (torch.zeros(372, dtype=torch.int64, device="cuda") for _ in range(2))
+    fpeer = torch.tensor([own.data_ptr(), peer.data_ptr()], dtype=torch.int64, device="cuda")
+    missing = torch.full((1,), -1, dtype=torch.int32, device="cuda")
+    own[0] = 1 << 20  # an epoch that neither counter reaches
+    ctx.quant_fp8_tensor(x, y, s, p, n)  # loads the code object
+    torch.cuda.synchronize()
+    p.zero_()
+    y.fill_(0x5a)
+    side, ended = torch.cuda.Stream(), torch.cuda.Event()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        arrive([own, fpeer, 1, 5, 2, missing], {})
+        ended.record()
+    marks = [torch.cuda.Event(enable_timing=True) for _ in range(9)]
+    marks[0].record()
+    for i in range(8):
+        ctx.quant_fp8_tensor(x, y, s, p, n)
+        marks[i + 1].record()
+    marks[8].synchronize()
+    waiting = not ended.query()
+    torch.cuda.synchronize()
+    us = sorted(marks[i].elapsed_time(marks[i + 1]) * 1e3 for i in range(8))
+    print(f"  the wave was still waiting: {waiting}; median {us[4]:.1f} us", flush=True)
+    assert int(missing[0]) == 0b11
+    assert torch.equal(p.view(torch.int32), want_p.view(torch.int32))
+    assert s.view(torch.int32).item() == want_s.view(torch.int32).item()
+    assert torch.equal(y, want_y)
+    assert us[4] < 200.0, us
+
+
+def test_quant_fp8_tensor_one_launch_in_a_graph(ctx):
+    """The one-launch form captured: every replay, on new inputs and with eager calls in
+    between, gives the pair's outputs (its partials are marked again each time)."""
+    n, nb = (24 << 20) + 5, 2048
+    print(f"[case] quant_fp8_tensor captured n={n}", flush=True)
+    x = torch.empty(n, dtype=torch.bfloat16, device="cuda")
+    y, want_y = (torch.empty(n, dtype=torch.uint8, device="cuda") for _ in range(2))
+    s, want_s = (torch.empty(1, dtype=torch.float32, device="cuda") for _ in range(2))
+    p, want_p = (torch.empty(nb, dtype=torch.float32, device="cuda") for _ in range(2))
+    x.fill_(1.0)
+    ctx.quant_fp8_tensor(x, y, s, p, n)  # loads the code object before capture
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ctx.quant_fp8_tensor(x, y, s, p, n)
+    stream = torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device="cuda").manual_seed(1600)
+    for r in range(4):
+        x.copy_(torch.empty(n, device="cuda").normal_(0, 2.0 / (r + 1), generator=g))
+        y.fill_(0x5a)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert ctx.L.k3h_quant_fp8_amax(ctx.h, stream, 1, x.data_ptr(), n, want_p.data_ptr(), nb) == 0
+        assert ctx.L.k3h_quant_fp8_apply(ctx.h, stream, 1, x.data_ptr(), want_y.data_ptr(), n,
+                                         want_p.data_ptr(), nb, want_s.data_ptr()) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(p.view(torch.int32), want_p.view(torch.int32)), f"replay {r}"
+        assert s.view(torch.int32).item() == want_s.view(torch.int32).item(), f"replay {r}"
+        assert torch.equal(y, want_y), f"replay {r}"
+    graph.reset()
