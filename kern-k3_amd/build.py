@@ -171,12 +171,19 @@ def build_host() -> str:
     return dst
 
 
-def build_py() -> str:
-    """The Python extension of k3h.py's tensor checks (host code, torch's C++ headers)."""
+def build_py() -> str | None:
+    """The Python extension of k3h.py's tensor checks (host code).  Without torch's C++
+    headers it is left out: the C library is whole without it."""
     import sysconfig
-
-    import torch
-    from torch.utils import cpp_extension
+    try:
+        import torch
+        from torch.utils import cpp_extension
+    except ImportError:
+        torch = None
+    if torch is None or not any(os.path.exists(os.path.join(p, "torch", "csrc", "autograd", "python_variable.h"))
+                                for p in cpp_extension.include_paths()):
+        print("[k3 build] no torch C++ headers: _k3h_py.so (k3h.py's calls) not built", flush=True)
+        return None
     dst = os.path.join(OUT, "_k3h_py.so")
     tmp = dst + ".tmp"
     tlib = os.path.join(os.path.dirname(torch.__file__), "lib")
@@ -218,7 +225,8 @@ def build(jobs: int | None = None, only: list[str] | None = None, oracle: bool =
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
         futs = [ex.submit(build_module, k) for k in keys]
         futs.append(ex.submit(build_host))
-        futs.append(ex.submit(build_py))
+        if not only:
+            futs.append(ex.submit(build_py))
         if oracle:
             futs.append(ex.submit(build_oracle))
         for f in futs:

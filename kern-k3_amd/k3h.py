@@ -160,23 +160,37 @@ def _check(rc: int, what: str) -> None:
 
 
 # ---------------------------------------------------------------- tensor checks
-def _load_checks():
-    """The extension built beside the library (csrc/host/k3h_py.cpp)."""
+# _dev(t, name, dtypes, numel=None, align=16) raises ValueError for anything but a
+# contiguous GPU tensor of one of dtypes (a sum of the masks below, the extension's DT_*
+# bits), at least numel elements and align-byte aligned; _ptr(t) is its address (None for None)
+BF16, F32, U8, I32, I64, ANY = 1, 2, 4 + 8, 16, 32, 0
+
+
+def _load_checks() -> None:
+    """Bind _dev and _ptr to the extension built beside the library (csrc/host/k3h_py.cpp)."""
+    global _dev, _ptr
     path = os.path.join(BUILD, "_k3h_py.so")
     if not os.path.exists(path):
         raise FileNotFoundError(f"{path} is missing: build it with `python kern-k3_amd/build.py`")
     spec = importlib.util.spec_from_file_location("_k3h_py", path)
     m = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(m)
-    return m
+    assert (BF16, F32, U8, I32, I64, ANY) == (m.BF16, m.F32, m.U8, m.I32, m.I64, m.ANY)
+    _dev, _ptr = m.dev, m.ptr
 
 
-_py = _load_checks()
-# _dev(t, name, dtypes, numel=None, align=16) raises ValueError for anything but a
-# contiguous GPU tensor of one of dtypes (a sum of the masks below), at least numel
-# elements and align-byte aligned; _ptr(t) is its address (None for None)
-_dev, _ptr = _py.dev, _py.ptr
-BF16, F32, U8, I32, I64, ANY = _py.BF16, _py.F32, _py.U8, _py.I32, _py.I64, _py.ANY
+def _dev(*args, **kw):  # not built when this file was imported
+    _load_checks()
+    return _dev(*args, **kw)
+
+
+def _ptr(t):
+    _load_checks()
+    return _ptr(t)
+
+
+if os.path.exists(os.path.join(BUILD, "_k3h_py.so")):
+    _load_checks()
 
 
 def _stream(stream: Any) -> int | None:

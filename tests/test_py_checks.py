@@ -1,10 +1,18 @@
 """The tensor checks of k3h.py's typed calls (extension _k3h_py): what a kernel argument is
 rejected for, on the CPU where the device decides first and on the GPU for the rest, and
 that a call runs on the stream current at that moment."""
+import importlib.util
+import os
+import shutil
+import subprocess
+import sys
+
 import pytest
 import torch
 
 import k3h
+
+PKG = os.path.dirname(os.path.abspath(k3h.__file__))
 
 
 def test_rejects_host_tensors_and_other_objects():
@@ -21,6 +29,54 @@ def test_rejects_host_tensors_and_other_objects():
     assert k3h._ptr(None) is None and k3h._ptr(t) == t.data_ptr()
     with pytest.raises(ValueError):
         k3h._ptr(3)
+
+
+def test_import_without_a_build(tmp_path):
+    """k3h.py imports where nothing is built; what needs the library or the extension names
+    the missing file, and the extension is picked up once it is there."""
+    shutil.copy(os.path.join(PKG, "k3h.py"), tmp_path)
+    code = f"""
+import os, shutil
+import k3h, torch
+assert os.path.dirname(os.path.abspath(k3h.__file__)) == {str(tmp_path)!r}
+assert k3h.pack_args(["i32"], [3]) == b"\\x03\\x00\\x00\\x00"
+for call in (k3h.Ctx, lambda: k3h._ptr(None), lambda: k3h._dev(torch.zeros(1), "x", k3h.F32)):
+    try:
+        call()
+    except FileNotFoundError as e:
+        assert "build.py" in str(e)
+    else:
+        raise SystemExit("no error without a build")
+os.makedirs(k3h.BUILD)
+shutil.copy({os.path.join(k3h.BUILD, "_k3h_py.so")!r}, k3h.BUILD)
+assert k3h._ptr(None) is None
+try:
+    k3h._dev(torch.zeros(1), "x", k3h.F32)
+except ValueError as e:
+    assert "must be a GPU tensor" in str(e)
+"""
+    env = dict(os.environ, PYTHONPATH=str(tmp_path))
+    r = subprocess.run([sys.executable, "-c", code], cwd=tmp_path, env=env, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+
+
+def test_library_builds_without_torch_headers(tmp_path, monkeypatch):
+    """The code objects and libk3h.so need no torch: `only=` leaves the extension alone, and a
+    whole build does without it where torch's C++ headers are missing."""
+    spec = importlib.util.spec_from_file_location("k3_build_headers", os.path.join(PKG, "build.py"))
+    b = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(b)
+    from torch.utils import cpp_extension
+    monkeypatch.setattr(b, "OUT", str(tmp_path))
+    monkeypatch.setattr(b, "MODULES", ["k3h_fused"])
+    ran = []
+    monkeypatch.setattr(b, "_run", lambda cmd, what: (ran.append(what), open(cmd[cmd.index("-o") + 1], "w").close()))
+    b.build(only=["k3h_fused"], oracle=False)
+    assert sorted(ran) == ["k3h_fused", "libk3h.so"]
+    ran.clear()
+    monkeypatch.setattr(cpp_extension, "include_paths", lambda *a, **k: [str(tmp_path)])
+    b.build(oracle=False)
+    assert sorted(ran) == ["k3h_fused", "libk3h.so"]
 
 
 @pytest.mark.gpu
