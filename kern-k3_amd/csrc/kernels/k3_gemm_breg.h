@@ -33,8 +33,10 @@
 // (39 tiles 71.9 against 72.0 us; with the rows known it would be 60).
 //
 // Cache policy: up to 1.25 tiles per expert the weights are loaded non-temporally (one
-// tile reads them: 101 -> 94 us at 39 tiles, 143 -> 132 at 56, 184 -> 178 at 63); above,
-// full tiles share them through the L2s (548 tiles: 1174 against 1430 us non-temporal).
+// tile reads them: 101 -> 94 us at 39 tiles, 143 -> 132 at 56, 184 -> 178 at 63); above, the
+// L2s serve an expert's second tile, full (548 tiles: 1174 against 1430 us non-temporal) or
+// thin (4000 tokens top-8, 91-99 tiles with thin last ones: 235 us where those loaded
+// non-temporally, 221 now; 6000 tokens 285 and 282).
 //
 // Measured and not kept: the persistent form of these items (two workgroups per CU, the
 // next item's A stages and scales requested during the current one's last steps): fc1
@@ -337,20 +339,24 @@ K3_DEV void k3b_run(const uint8_t* __restrict__ a, const uint8_t* __restrict__ a
   // stream them faster; with more, the L2s serve the second tile.
   const int live = *num_tiles;
   const bool once = live <= E + E / 4;
-  if (need <= 32) {
-    k3_v16f acc[1][2];
-    k3b_loop<1, 6, 8, 16, true>(acc, a, a_sf, v0, v1, wb0, wb1, sbu, K, w, lane);
-    epi(acc, std::integral_constant<int, 1>{}, tile, cb, e, w, lane);
-  } else if (need <= 64) {
-    k3_v16f acc[2][2];
-    k3b_loop<2, 6, 6, 8, true>(acc, a, a_sf, v0, v1, wb0, wb1, sbu, K, w, lane);
-    epi(acc, std::integral_constant<int, 2>{}, tile, cb, e, w, lane);
-  } else {
-    k3_v16f acc[4][2];
-    if (once) k3b_loop<4, 2, 3, 4, true>(acc, a, a_sf, v0, v1, wb0, wb1, sbu, K, w, lane);
-    else k3b_loop<4, 2, 3, 4, false>(acc, a, a_sf, v0, v1, wb0, wb1, sbu, K, w, lane);
-    epi(acc, std::integral_constant<int, 4>{}, tile, cb, e, w, lane);
-  }
+  auto item = [&](auto mt_c, auto nb_c, auto pa_c, auto rs_c) {
+    constexpr int MT = decltype(mt_c)::value, NB = decltype(nb_c)::value;
+    constexpr int PA = decltype(pa_c)::value, RS = decltype(rs_c)::value;
+    k3_v16f acc[MT][2];
+    if (once) k3b_loop<MT, NB, PA, RS, true>(acc, a, a_sf, v0, v1, wb0, wb1, sbu, K, w, lane);
+    else k3b_loop<MT, NB, PA, RS, false>(acc, a, a_sf, v0, v1, wb0, wb1, sbu, K, w, lane);
+    epi(acc, mt_c, tile, cb, e, w, lane);
+  };
+  using std::integral_constant;
+  if (need <= 32)
+    item(integral_constant<int, 1>{}, integral_constant<int, 6>{}, integral_constant<int, 8>{},
+         integral_constant<int, 16>{});
+  else if (need <= 64)
+    item(integral_constant<int, 2>{}, integral_constant<int, 6>{}, integral_constant<int, 6>{},
+         integral_constant<int, 8>{});
+  else
+    item(integral_constant<int, 4>{}, integral_constant<int, 2>{}, integral_constant<int, 3>{},
+         integral_constant<int, 4>{});
 }
 
 // bf16 out, stored as by k3w_gemm_bf16.

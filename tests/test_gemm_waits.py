@@ -90,4 +90,22 @@ def test_counted_waits_count_issued_loads(listing, entry):
         assert steps[-1][4] == [mt, 3], steps
         # its own second weights are among the loads of len(steps) - 1 whole steps and two
         assert {w for *_, w, _ in steps} == {first[3]} and first[3] <= 2 + (len(steps) - 1) * (5 + mt)
-    assert sorted({s[0][2] // 2 for s in loops}) == [1, 2, 4]
+    assert sorted(s[0][2] // 2 for s in loops) == [1, 1, 2, 2, 4, 4]
+
+
+@pytest.mark.parametrize("entry", ENTRIES)
+def test_every_tile_height_has_both_weight_policies(listing, entry):
+    """Non-temporal weights up to 1.25 tiles per expert, cacheable ones above, for tiles of
+    one, two and four m tiles alike."""
+    bodies, mfma, loads, nt = set(), 0, 0, 0
+    for s in listing[entry]:
+        if s.startswith("v_mfma"):
+            mfma += 1
+        elif s.startswith("global_load_dwordx4"):
+            loads += 1
+            nt += s.endswith(" nt")
+        elif s.startswith("s_barrier"):
+            if mfma in (4, 8, 16) and loads == 4:  # a whole step of the K loop
+                bodies.add((mfma // 4, nt > 0))
+            mfma = loads = nt = 0
+    assert bodies == {(mt, policy) for mt in (1, 2, 4) for policy in (False, True)}, bodies

@@ -291,13 +291,15 @@ def test_wide_items_match_4wave(ctx, K):
             assert same
 
 
+@pytest.mark.parametrize("E", [3, 16])
 @pytest.mark.parametrize("K", [512, 768, 1024, 3584])
-def test_repeated_rows_match_gathered(ctx, K):
+def test_repeated_rows_match_gathered(ctx, K, E):
     """Tiles padded by repeating a row index (the fc1 kernel computes one or two m tiles
     and repeats the last row's results) against the same rows gathered beforehand
     (a_rows = None, every row computed), bit for bit: distinct rows on both sides of each
-    m tile's edge, a repeat of a live row's index, and index -1 (row 0)."""
-    E, inter = 3, 256
+    m tile's edge, a repeat of a live row's index, and index -1 (row 0); with fewer experts
+    than tiles (cacheable weights) and with more (non-temporal)."""
+    inter = 256
     N = 2 * inter
     _case(f"repeated rows E={E} inter={inter} K={K}")
     g, q, sf, w, wsf = _inputs(7900 + K, 300, E, N, K, wsf_range=(121, 126))
