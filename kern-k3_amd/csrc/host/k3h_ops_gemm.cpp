@@ -20,8 +20,6 @@ constexpr int kTileN = 256, kTileNWide = 512, kStepK = 128;
 // The kernels keep the tile's A scales (K / 32 bytes per row) in LDS: entries
 // without a suffix take K <= 3584, the "_w" entries K <= 7168.
 constexpr int kMaxK = 7168, kMaxKNarrow = 3584;
-// The kernels' split of the 256-column items over the XCDs (K3G_XT x K3G_XC).
-constexpr int kXt = 4, kXc = 2;
 
 bool gemm_shape_ok(int E, int N, int K, int max_tiles) {
   return E > 0 && N > 0 && K > 0 && max_tiles >= 0 && N % kTileN == 0 && K % kStepK == 0 &&
@@ -149,45 +147,25 @@ K3H_API int k3h_moe_gemm_mx(k3h_ctx_t ctx, void* stream, int epilogue, const voi
   // per turn, at least four steps for the loads in flight, A scales of K <= 3584
   const bool breg = K % (2 * kStepK) == 0 && K >= 4 * kStepK && K <= kMaxKNarrow;
   const uint32_t rows = gemm_grid_rows(max_tiles, N / kTileN);
+  // bf16 with hardly a row per expert (max_tiles counts a partial tile for each): the
+  // weights' stream bounds it, and 256-column items on two workgroups per CU stream them
+  // faster as long as they fit about one round (1 tile 29 -> 22 us, 39 tiles 86 -> 68, but 56
+  // tiles 93 -> 96)
+  if (epilogue == K3H_GEMM_BF16 && breg && max_tiles <= E + E / 16 && rows <= 65535u)
+    return k3h_run(ctx, "k3h_moe_gemm", "kern_k3h_moe_gemm3_bf16", (uint32_t)(N / kTileN), rows, 1,
+                   kBlock, stream, args);
   // f32 / bf16 epilogues on 512-column items: persistent 8-wave workgroups
   // (kern_k3h_moe_gemm2_*, one per CU, grid a multiple of the 8 XCDs) where the
   // shape allows them; else, and for the SiTU-GLU + MXFP8 epilogue and its f32 tiling, 256-column
   // items on 4-wave workgroups (two per CU).
-  const bool wide_items = (epilogue == K3H_GEMM_F32 || epilogue == K3H_GEMM_BF16) &&
-                          N % kTileNWide == 0 && K >= 2 * kStepK && K <= kMaxKNarrow &&
-                          k3h_aligned(out, 16);
-  int cus = 0;
-  if (wide_items) {
+  if ((epilogue == K3H_GEMM_F32 || epilogue == K3H_GEMM_BF16) && N % kTileNWide == 0 && K >= 2 * kStepK &&
+      K <= kMaxKNarrow && k3h_aligned(out, 16)) {
+    int cus = 0;
     if (const int rc = stream_cus(stream, &cus)) return rc;
-    cus = std::max(8, cus / 8 * 8);
-  }
-  // bf16 over few tiles, where the weights' stream bounds it, on register-weight items too:
-  // * one of them per CU at most, whatever the live count: the CUs that 512-column items
-  //   leave idle (16 tiles x 14 blocks 36 -> 27 us, 8 x 14 33 -> 22, 64 x 4 38 -> 31, 64 x 2 35
-  //   -> 25; with as many blocks as CUs 38.9 -> 30.3, and 38.9 -> 39.7 for 128 tiles x 2);
-  // * hardly a row per expert (max_tiles counts a partial tile for each): the live tiles are
-  //   far fewer and only the device knows them, so both forms are launched and
-  //   k3g_narrow_rounds lets one of them work (the other's launch: 1.3 to 2.5 us);
-  // * N without 512-column items: against the 256-column items in LDS 1.02 to 1.38 times as
-  //   fast at 1 to 238 tiles.
-  int both = 0;  // the CU count that k3g_narrow_rounds decides by
-  if (epilogue == K3H_GEMM_BF16 && breg && rows <= 65535u) {
-    const int64_t share = (int64_t)k3h_cdiv(max_tiles, kXt) * k3h_cdiv(N / kTileN, kXc);
-    const bool one = wide_items && share * 8 <= cus;
-    if (one || max_tiles <= E + E / 16) {
-      both = wide_items && !one ? cus : 0;
-      K3hArgs narrow = args;
-      narrow.i32(both);
-      const int rc = k3h_run(ctx, "k3h_moe_gemm", "kern_k3h_moe_gemm3_bf16",
-                             (uint32_t)(N / kTileN), rows, 1, kBlock, stream, narrow);
-      if (rc != K3H_OK || !both) return rc;
-    }
-  }
-  if (wide_items) {
-    if (epilogue == K3H_GEMM_BF16) args.i32(both);
+    const uint32_t grid = (uint32_t)std::max(8, cus / 8 * 8);
     return k3h_run(ctx, "k3h_moe_gemm",
                    epilogue == K3H_GEMM_F32 ? "kern_k3h_moe_gemm2_f32" : "kern_k3h_moe_gemm2_bf16",
-                   (uint32_t)cus, 1, 1, kBlockWide, stream, args);
+                   grid, 1, 1, kBlockWide, stream, args);
   }
   if (rows > 65535u) return K3H_EINVAL;
   if (breg && epilogue == K3H_GEMM_SITU_MX) entry = "kern_k3h_moe_gemm3_situ_mx";

@@ -498,8 +498,7 @@ K3_DEV void k3b_gemm_acc(K3G_PARAMS, float* __restrict__ out) {
     k3b_gemm_acc(K3G_ARGS, out);                                                                 \
   }                                                                                              \
   extern "C" __global__ void __launch_bounds__(256, 2)                                           \
-      kern_k3h_moe_gemm3_bf16(K3G_PARAMS, uint16_t* __restrict__ out, int cus) {                 \
-    if (cus && !k3g_narrow_rounds(num_tiles, max_tiles, N, cus)) return;                         \
+      kern_k3h_moe_gemm3_bf16(K3G_PARAMS, uint16_t* __restrict__ out) {                          \
     k3b_gemm_bf16(K3G_ARGS, out);                                                                \
   }                                                                                              \
   extern "C" __global__ void __launch_bounds__(256, 2)                                           \

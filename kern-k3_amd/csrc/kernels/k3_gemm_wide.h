@@ -423,15 +423,12 @@ K3_DEV void k3w_gemm_bf16(K3G_PARAMS, uint16_t* __restrict__ out) {
   });
 }
 
-// kern_k3h_moe_gemm2_bf16 with cus != 0 leaves its items to kern_k3h_moe_gemm3_bf16, launched
-// beside it, where k3g_narrow_rounds says so.
 #define K3W_ENTRIES                                                                              \
   extern "C" __global__ void __launch_bounds__(512, 1)                                           \
       kern_k3h_moe_gemm2_f32(K3G_PARAMS, float* __restrict__ out) {                              \
     k3w_gemm_f32(K3G_ARGS, out);                                                                 \
   }                                                                                              \
   extern "C" __global__ void __launch_bounds__(512, 1)                                           \
-      kern_k3h_moe_gemm2_bf16(K3G_PARAMS, uint16_t* __restrict__ out, int cus) {                 \
-    if (cus && k3g_narrow_rounds(num_tiles, max_tiles, N, cus)) return;                          \
+      kern_k3h_moe_gemm2_bf16(K3G_PARAMS, uint16_t* __restrict__ out) {                          \
     k3w_gemm_bf16(K3G_ARGS, out);                                                                \
   }

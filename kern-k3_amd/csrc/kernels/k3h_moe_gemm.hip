@@ -462,22 +462,6 @@ K3_DEV bool k3g_item(const int* __restrict__ num_tiles, int max_tiles, int& tile
   return true;
 }
 
-// Whether the live tiles' bf16 products take fewer rounds, weighted by what a round costs,
-// on 256-column register-weight items (kern_k3h_moe_gemm3_bf16, two workgroups per CU) than
-// on 512-column ones (kern_k3h_moe_gemm2_bf16, one per CU).  A round here is one item per CU
-// of an XCD: about 24 us of the first (the largest XCD's share counts) and 45 us of the
-// second, at K = 3072 with every tile its own expert.  Measured, 256- / 512-column items in
-// us, N = 3584: 8 tiles 24 / 31, 16 27 / 36, 20 44 / 39, 36 58 / 54, 39 71 / 80, 50 75 / 87,
-// 56 92 / 93, 74 117 / 135, 150 219 / 238; N = 7168: 18 69 / 49, 20 68 / 82, 39 118 / 135.
-K3_DEV bool k3g_narrow_rounds(const int* __restrict__ num_tiles, int max_tiles, int N, int cus) {
-  int live = *num_tiles;
-  live = live < max_tiles ? live : max_tiles;
-  const int nc = N / K3G_TILE_N, per_xcd = cus / K3G_XCDS;
-  const int share = (live + K3G_XT - 1) / K3G_XT * ((nc + K3G_XC - 1) / K3G_XC);
-  const int r3 = (share + per_xcd - 1) / per_xcd, r2 = (live * nc + 2 * cus - 1) / (2 * cus);
-  return r3 < 2 * r2;
-}
-
 // Accumulates the wave's 64 x 128 block of work item (tile, cb); returns false
 // when the tile's expert is out of range (the whole workgroup skips the item).
 template <int KGM, bool SW>

@@ -358,50 +358,3 @@ def test_bf16_few_tiles_match_many(ctx, N, K, gather):
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
     assert (outs[0][3 * 128:4 * 128] == 7).all() and (outs[0][nt * 128:] == 7).all()
     assert not (outs[0][:3 * 128] == 7).all()
-
-
-def _narrow_rounds(live, N, cus):
-    """k3g_narrow_rounds: 256-column items take fewer weighted rounds than 512-column ones."""
-    nc, per_xcd = N // 256, cus // 8
-    share = -(-live // 4) * -(-nc // 2)
-    return -(-share // per_xcd) < 2 * -(-live * nc // (2 * cus))
-
-
-@pytest.mark.parametrize("N,live", [(512, 1), (1024, 64), (1024, 65), (3584, 0), (3584, 1), (3584, 16),
-                                    (3584, 17), (3584, 36), (3584, 37), (3584, 52), (3584, 53),
-                                    (7168, 8), (7168, 9), (7168, 18), (7168, 19)])
-def test_bf16_one_of_two_forms_by_the_live_count(ctx, N, live):
-    """bf16 output over at most E + E / 16 tiles: of the two forms that are launched, the
-    device's live count picks one by its rounds (both sides of each change of the pick at
-    256 CUs), and the typed call stores the same bits as the form for more tiles."""
-    import ctypes
-    import k3h
-    E, K, max_tiles = 64, 512, 68
-    cus = torch.cuda.get_device_properties(0).multi_processor_count // 8 * 8
-    _case(f"bf16 by live count N={N} live={live} cus={cus}")
-    g, q, sf, w, wsf = _inputs(8300 + N + live, max_tiles * 128, E, N, K)
-    cta = np.concatenate([g.permutation(max_tiles)[:live] % E, np.zeros(max_tiles - live)]).astype(np.int32)
-    wt, st = _tiled(ctx, w, wsf, E, N, K, 0)
-    da, dsf, dnt, dcta = to_dev(q), to_dev(sf), to_dev(np.array([live], np.int32)), to_dev(cta)
-    outs = {}
-    for form, entry, grid, block, gate in (
-            ("narrow", "kern_k3h_moe_gemm3_bf16", (N // 256, _grid_rows(max_tiles, N // 256), 1), 256, cus),
-            ("wide", "kern_k3h_moe_gemm2_bf16", (cus, 1, 1), 512, cus),
-            ("all wide", "kern_k3h_moe_gemm2_bf16", (cus, 1, 1), 512, 0)):
-        outs[form] = torch.full((max_tiles * 128, N), 7.0, dtype=torch.bfloat16, device="cuda")
-        args = k3h.pack_args(["buffer"] * 7 + ["i32"] * 4 + ["buffer", "i32"],
-                             [da, dsf, None, wt, st, dnt, dcta, E, N, K, max_tiles, outs[form], gate])
-        cbuf = ctypes.create_string_buffer(args, len(args))
-        k3h._check(ctx.L.k3h_launch(ctx.function("k3h_moe_gemm", entry), (ctypes.c_uint32 * 3)(*grid),
-                                    (ctypes.c_uint32 * 3)(block, 1, 1), 0, None,
-                                    ctypes.cast(cbuf, ctypes.c_void_p), len(args)), entry)
-    typed = torch.full_like(outs["wide"], 7.0)
-    ctx.moe_gemm_mx(ctx.GEMM_BF16, da, dsf, None, wt, st, dnt, dcta, max_tiles, E, N, K, typed)
-    torch.cuda.synchronize()
-    want = outs["all wide"]
-    narrow = live > 0 and _narrow_rounds(live, N, cus)
-    for form, works in (("narrow", narrow), ("wide", not narrow)):
-        exp = want if works else torch.full_like(want, 7.0)
-        assert torch.equal(outs[form].view(torch.int16), exp.view(torch.int16)), form
-    assert torch.equal(typed.view(torch.int16), want.view(torch.int16))
-    assert (want[live * 128:] == 7).all() and (live == 0 or not (want[:live * 128] == 7).all())
