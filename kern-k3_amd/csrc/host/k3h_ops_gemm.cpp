@@ -20,6 +20,8 @@ constexpr int kTileN = 256, kTileNWide = 512, kStepK = 128;
 // The kernels keep the tile's A scales (K / 32 bytes per row) in LDS: entries
 // without a suffix take K <= 3584, the "_w" entries K <= 7168.
 constexpr int kMaxK = 7168, kMaxKNarrow = 3584;
+// The kernels' split of the 256-column items over the XCDs (K3G_XT x K3G_XC).
+constexpr int kXt = 4, kXc = 2;
 
 bool gemm_shape_ok(int E, int N, int K, int max_tiles) {
   return E > 0 && N > 0 && K > 0 && max_tiles >= 0 && N % kTileN == 0 && K % kStepK == 0 &&
@@ -147,26 +149,42 @@ K3H_API int k3h_moe_gemm_mx(k3h_ctx_t ctx, void* stream, int epilogue, const voi
   // per turn, at least four steps for the loads in flight, A scales of K <= 3584
   const bool breg = K % (2 * kStepK) == 0 && K >= 4 * kStepK && K <= kMaxKNarrow;
   const uint32_t rows = gemm_grid_rows(max_tiles, N / kTileN);
-  // bf16 with hardly a row per expert (max_tiles counts a partial tile for each): the
-  // weights' stream bounds it, and 256-column items on two workgroups per CU stream them
-  // faster as long as they fit about one round (1 tile 29 -> 22 us, 39 tiles 86 -> 68, but 56
-  // tiles 93 -> 96)
-  if (epilogue == K3H_GEMM_BF16 && breg && max_tiles <= E + E / 16 && rows <= 65535u)
-    return k3h_run(ctx, "k3h_moe_gemm", "kern_k3h_moe_gemm3_bf16", (uint32_t)(N / kTileN), rows, 1,
-                   kBlock, stream, args);
   // f32 / bf16 epilogues on 512-column items: persistent 8-wave workgroups
   // (kern_k3h_moe_gemm2_*, one per CU, grid a multiple of the 8 XCDs) where the
   // shape allows them; else, and for the SiTU-GLU + MXFP8 epilogue and its f32 tiling, 256-column
   // items on 4-wave workgroups (two per CU).
-  if ((epilogue == K3H_GEMM_F32 || epilogue == K3H_GEMM_BF16) && N % kTileNWide == 0 && K >= 2 * kStepK &&
-      K <= kMaxKNarrow && k3h_aligned(out, 16)) {
-    int cus = 0;
+  const bool wide_items = (epilogue == K3H_GEMM_F32 || epilogue == K3H_GEMM_BF16) &&
+                          N % kTileNWide == 0 && K >= 2 * kStepK && K <= kMaxKNarrow &&
+                          k3h_aligned(out, 16);
+  int cus = 0;
+  if (wide_items) {
     if (const int rc = stream_cus(stream, &cus)) return rc;
-    const uint32_t grid = (uint32_t)std::max(8, cus / 8 * 8);
+    cus = std::max(8, cus / 8 * 8);
+  }
+  // bf16 over few tiles, where the weights' stream bounds it, on register-weight items:
+  // * at most one per CU, whatever the live count is: 512-column items leave at least half
+  //   of the CUs idle (K = 3072, tiles x column blocks: 8 x 14 33 -> 22 us, 16 x 14 36 -> 27,
+  //   64 x 4 38 -> 31, 64 x 2 35 -> 25; with as many items as CUs 16 x 16 39 -> 30, but 128 x 2
+  //   38.9 -> 39.7);
+  // * hardly a row per expert (max_tiles counts a partial tile for each), where the live
+  //   tiles are fewer, how many is known on the device only.  The wide items' time jumps
+  //   with each round of 2 x CUs blocks, the narrow ones' with each item per CU (256 CUs, E =
+  //   56, N = 3584, wide -> narrow): 1 tile 28 -> 21 us, 16 36 -> 28, 20 38 -> 43, 36 51 -> 55,
+  //   39 85 -> 70, 52 89 -> 75, 56 92 -> 92, 59 91 -> 94; N = 7168: 18 tiles 51 -> 69, 20 82 ->
+  //   70, 56 185 -> 167.  Launching both and letting the live count pick cost 2 to 4 us a call
+  //   (39 tiles 74) and gave 2 to 4 at 17 to 36 tiles: not kept;
+  // * N without 512-column items: against the 256-column items in LDS 1.02 to 1.38 times as
+  //   fast at 1 to 238 tiles.
+  if (epilogue == K3H_GEMM_BF16 && breg && rows <= 65535u) {
+    const int64_t share = (int64_t)k3h_cdiv(max_tiles, kXt) * k3h_cdiv(N / kTileN, kXc);
+    if ((wide_items && share * 8 <= cus) || max_tiles <= E + E / 16)
+      return k3h_run(ctx, "k3h_moe_gemm", "kern_k3h_moe_gemm3_bf16", (uint32_t)(N / kTileN), rows, 1,
+                     kBlock, stream, args);
+  }
+  if (wide_items)
     return k3h_run(ctx, "k3h_moe_gemm",
                    epilogue == K3H_GEMM_F32 ? "kern_k3h_moe_gemm2_f32" : "kern_k3h_moe_gemm2_bf16",
-                   grid, 1, 1, kBlockWide, stream, args);
-  }
+                   (uint32_t)cus, 1, 1, kBlockWide, stream, args);
   if (rows > 65535u) return K3H_EINVAL;
   if (breg && epilogue == K3H_GEMM_SITU_MX) entry = "kern_k3h_moe_gemm3_situ_mx";
   if (breg && epilogue == K3H_GEMM_F32_SITU_TILING) entry = "kern_k3h_moe_gemm3_acc";

@@ -358,3 +358,32 @@ def test_bf16_few_tiles_match_many(ctx, N, K, gather):
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
     assert (outs[0][3 * 128:4 * 128] == 7).all() and (outs[0][nt * 128:] == 7).all()
     assert not (outs[0][:3 * 128] == 7).all()
+
+
+@pytest.mark.parametrize("N,K,max_tiles", [(512, 512, 125), (512, 768, 129), (3584, 1024, 16),
+                                           (3584, 512, 17), (1024, 512, 61), (7168, 512, 8)])
+def test_bf16_one_round_matches_wide(ctx, N, K, max_tiles):
+    """bf16 output with few experts: up to one 256-column item per CU the typed call takes the
+    register-weight items however many tiles an expert has, here on both sides of that at
+    256 CUs, against the 512-column entry launched directly, bit for bit, all tiles live."""
+    import ctypes
+    import k3h
+    E = 6
+    _case(f"bf16 one round N={N} K={K} tiles={max_tiles}")
+    g, q, sf, w, wsf = _inputs(8400 + N + max_tiles, max_tiles * 128, E, N, K)
+    cta = np.sort(g.integers(0, E, max_tiles)).astype(np.int32)
+    wt, st = _tiled(ctx, w, wsf, E, N, K, 0)
+    da, dsf, dnt, dcta = to_dev(q), to_dev(sf), to_dev(np.array([max_tiles], np.int32)), to_dev(cta)
+    got, want = (torch.full((max_tiles * 128, N), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    ctx.moe_gemm_mx(ctx.GEMM_BF16, da, dsf, None, wt, st, dnt, dcta, max_tiles, E, N, K, got)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count // 8 * 8
+    args = k3h.pack_args(["buffer"] * 7 + ["i32"] * 4 + ["buffer"],
+                         [da, dsf, None, wt, st, dnt, dcta, E, N, K, max_tiles, want])
+    cbuf = ctypes.create_string_buffer(args, len(args))
+    entry = "kern_k3h_moe_gemm2_bf16"
+    k3h._check(ctx.L.k3h_launch(ctx.function("k3h_moe_gemm", entry), (ctypes.c_uint32 * 3)(cus, 1, 1),
+                                (ctypes.c_uint32 * 3)(512, 1, 1), 0, None,
+                                ctypes.cast(cbuf, ctypes.c_void_p), len(args)), entry)
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    assert not (want == 7).all(1).any()
