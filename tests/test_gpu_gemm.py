@@ -287,15 +287,28 @@ def test_wide_items_match_4wave(ctx, K):
                             K, fc1t)
             torch.cuda.synchronize()
             same = torch.equal(got.view(torch.uint8), fc1t.view(torch.uint8))
-            print(f"  kern_k3h_moe_gemm_situ_acc: identical = {same}", flush=True)
+            breg = K % 256 == 0 and 512 <= K <= 3584  # the register-weight items' range
+            print(f"  kern_k3h_moe_gemm{'3_acc' if breg else '_situ_acc'}: identical = {same}", flush=True)
             assert same
+            if breg:  # the 256-column form, which other K take
+                fc1t.fill_(fill)
+                entry = "kern_k3h_moe_gemm_situ_acc"
+                args = k3h.pack_args(["buffer"] * 7 + ["i32"] * 4 + ["buffer"],
+                                     [dq, dsf, dr, wt, st, nt, dcta, E, N, K, max_tiles, fc1t])
+                cbuf = ctypes.create_string_buffer(args, len(args))
+                k3h._check(ctx.L.k3h_launch(ctx.function("k3h_moe_gemm", entry), grid, block, 0, None,
+                                            ctypes.cast(cbuf, ctypes.c_void_p), len(args)), entry)
+                torch.cuda.synchronize()
+                same = torch.equal(got.view(torch.uint8), fc1t.view(torch.uint8))
+                print(f"  {entry}: identical = {same}", flush=True)
+                assert same
 
 
 @pytest.mark.parametrize("E", [3, 16])
 @pytest.mark.parametrize("K", [512, 768, 1024, 3584])
 def test_repeated_rows_match_gathered(ctx, K, E):
-    """Tiles padded by repeating a row index (the fc1 kernel computes one or two m tiles
-    and repeats the last row's results) against the same rows gathered beforehand
+    """Tiles padded by repeating a row index (the register-weight items compute one or two m
+    tiles and repeat the last row's results: SiTU, f32 and bf16 output) against the same rows gathered beforehand
     (a_rows = None, every row computed), bit for bit: distinct rows on both sides of each
     m tile's edge, a repeat of a live row's index, and index -1 (row 0); with fewer experts
     than tiles (cacheable weights) and with more (non-temporal)."""
@@ -326,9 +339,17 @@ def test_repeated_rows_match_gathered(ctx, K, E):
         ctx.moe_gemm_mx(ctx.GEMM_F32_SITU_TILING, da, dasf, idx, wt, st, dnt, dcta, nt, E, N, K, acc)
         ctx.moe_gemm_mx(ctx.GEMM_SITU_MX, da, dasf, idx, wt, st, dnt, dcta, nt, E, N, K, oq, osf,
                         alpha, beta)
+        # bf16 output: its own broadcast of the last row (exchanged lanes); the typed call takes
+        # the same entry (at most one item per CU)
+        ob = torch.full((nt * 128, N), 7.0, dtype=torch.bfloat16, device="cuda")
+        ctx.moe_gemm_mx(ctx.GEMM_BF16, da, dasf, idx, wt, st, dnt, dcta, nt, E, N, K, ob)
         torch.cuda.synchronize()
-        got.append((from_dev(acc).view(np.uint32), from_dev(oq), from_dev(osf)))
-    for name, x, y in zip(("accumulators", "codes", "scales"), *got):
+        got.append((from_dev(acc).view(np.uint32), from_dev(oq), from_dev(osf),
+                    ob.view(torch.int16).cpu().numpy()))
+    # and the values of the f32 accumulators: their RNE bf16 rounding
+    bf = torch.from_numpy(got[1][0].view(np.float32)).to(torch.bfloat16).view(torch.int16).numpy()
+    assert np.array_equal(got[1][3].reshape(bf.shape), bf)
+    for name, x, y in zip(("accumulators", "codes", "scales", "bf16"), *got):
         bad = (x.reshape(nt, -1) != y.reshape(nt, -1)).any(1)
         assert not bad.any(), f"{name}: tiles {np.flatnonzero(bad)} differ"
 
@@ -341,7 +362,7 @@ def test_bf16_few_tiles_match_many(ctx, N, K, gather):
     out of range, keep their rows."""
     E = 16
     _case(f"bf16 few tiles E={E} N={N} K={K} gather={gather}")
-    few, many, nt = 17, 40, 15
+    few, many, nt = 17, 132 if N == 512 else 40, 15  # many: more than one item per CU
     g, q, sf, w, wsf = _inputs(8100 + N + K, many * 128, E, N, K)
     cta = g.permutation(E)[:nt].astype(np.int32)
     cta[3] = E
