@@ -338,8 +338,8 @@ def _bench_ops(ctx, reps: int, out_path: str | None, cpu_budget: float = 0.0, gr
     sc = torch.empty(1, dtype=torch.float32, device="cuda")
     parts = torch.empty(2048, dtype=torch.float32, device="cuda")
     add("per-tensor fp8 pair (amax+apply)", "k3h_quant_fp8_{mark,once}", f"{T}x{H}",
-        2 * T * H * 2 + T * H, timed(lambda: ctx.quant_fp8_tensor(x, q, sc, parts, T * H, stream=s)),
-        note="one launch keeps 98 MB of x on the chip; the rest is read again from the MALL",
+        T * H * 2 + T * H, timed(lambda: ctx.quant_fp8_tensor(x, q, sc, parts, T * H, stream=s)),
+        note="x counted once; one launch keeps 100.7 MB of it on the chip and reads the rest again from the MALL",
         cpu=O and (lambda: O.quant_fp8_apply(xh, T * H, O.quant_fp8_amax(xh, T * H, 2048), 2048)))
     del xh
     del ro, q, sf

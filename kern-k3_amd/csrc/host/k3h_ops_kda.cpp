@@ -32,8 +32,8 @@ K3H_API int k3h_span_gather(k3h_ctx_t ctx, void* stream, const void* partial, co
   // taps pass through LDS): one work item per (tile pair, stream, column tile)
   // and one beta / flow item per tile pair, as a 1-D grid.  The entry also runs
   // the manifest's (INNER / 512, 4, ceil(span / 16)) x 128 geometry.
-  // Short spans take 4-row tiles: kernel time 16 rows 4.9 -> 3.3 us, 300 5.8 -> 5.0, 517
-  // 7.4 -> 7.1, 800 8.3 -> 9.9 (the re-read tap rows).
+  // Short spans take 4-row tiles: back to back 517 rows 8.17 -> 7.67 us, 600 8.52 -> 8.48, 700
+  // 8.68 -> 9.32 (the re-read tap rows).
   const bool is_short = span <= kSpanShort;
   const uint32_t pairs = k3h_cdiv(k3h_cdiv(span, is_short ? 4 : 16), kSpanShare);
   return k3h_run(ctx, "k3_span_gather_v3+HEADS=24",

@@ -2,7 +2,7 @@
 // k3h_moe_gemm.hip after the 256-column kernels and k3_gemm_wide.h, whose layouts,
 // item split and helpers it shares).  Entries kern_k3h_moe_gemm3_situ_mx (fc1),
 // kern_k3h_moe_gemm3_acc (its tiling with f32 output) and kern_k3h_moe_gemm3_bf16 (fc2 over
-// few tiles): the same products as the 256-column kernels bit for bit (the same MFMA
+// few tiles, by k3h_moe_gemm_mx's rule): the same products as the 256-column kernels bit for bit (the same MFMA
 // sequence per output element), for 512 <= K <= 3584, K % 256 == 0.
 //
 // Work item: route tile t (128 rows) x one 256-column block, one 256-thread
@@ -27,10 +27,10 @@
 // (39 tiles 95.6 us at four / five steps, 91.2 at six; 56 tiles 133.4 -> 127; eight
 // steps no faster).
 //
-// Without a row list (fc2) every row is computed.  There the A rows, not their MFMAs, are
-// the cost: 16 KB per step and workgroup, as many bytes as the weights.  Finding the
-// repeated rows by comparing them on the way reads them all the same and gains nothing
-// (39 tiles 71.9 against 72.0 us; with the rows known it would be 60).
+// Without a row list (fc2) every row is computed.  Finding the repeated rows by comparing
+// them on the way reads them all the same and gains nothing (39 tiles 71.9 against 72.0 us;
+// with the rows known it would be 60: the routing's cta_limit holds them, but the call has no
+// parameter for it).
 //
 // Cache policy: up to 1.25 tiles per expert the weights are loaded non-temporally (one
 // tile reads them: 101 -> 94 us at 39 tiles, 143 -> 132 at 56, 184 -> 178 at 63); above, the

@@ -84,7 +84,7 @@ K3_DEV k3_u2 k9_row(const float* a0, const float* a1, const float* a2, const flo
 
 K3_DEV k3_u2 k9_ld8_nt(const uint16_t* p) { return __builtin_nontemporal_load((const k3_u2*)p); }
 
-#define K9_SHARE_MAX 4  // 16-row tiles per workgroup (block 128 x share)
+#define K9_SHARE_MAX 4  // row tiles (16 or 4 rows) per workgroup (block 128 x share)
 
 #define K9_PARAMS                                                                             \
   const uint16_t *__restrict__ partial, const float *__restrict__ cw,                        \
@@ -227,8 +227,10 @@ extern "C" __global__ void __launch_bounds__(128 * K9_SHARE_MAX) kern_k3_span_ga
 
 // Short spans: 4-row tiles.  With 16 a span of a few hundred rows has fewer waves than the
 // chip has SIMDs, and each of them evaluates 64 activations one after another; the tap
-// rows that shorter tiles read again come from the L2s (kernel time 16 rows 4.9 -> 3.3 us,
-// 300 5.8 -> 5.0, 517 7.4 -> 7.1, 800 8.3 -> 9.9: the typed call takes it up to 600 rows).
+// rows that shorter tiles read again come from the L2s.  The typed call takes them up to 600
+// rows (kernel time 16 rows 5.3 -> 4.0 us, 300 6.6 -> 6.1; back to back over twelve buffer
+// sets 400 rows 6.72 -> 6.63 us, 517 8.17 -> 7.67, 560 8.38 -> 7.86, 600 8.52 -> 8.48, 640 8.57
+// -> 8.48, 700 8.68 -> 9.32, 800 8.85 -> 10.0; 440 6.88 -> 6.99).
 extern "C" __global__ void __launch_bounds__(128 * K9_SHARE_MAX) k3h_span_gather_short(K9_PARAMS) {
   k9_span_gather<4>(partial, cw, kda_base, line_index, line_bytes, wsm_partial, span_q, span_k,
                     span_v, span_beta, span_flow, span_at, span);
